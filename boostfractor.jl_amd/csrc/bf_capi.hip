@@ -163,6 +163,7 @@ int bf_ctx_destroy(bf_ctx* ctx) {
     (void)hipStreamSynchronize(ctx->stream);
     bf::clear_timers(ctx);
     ctx->twiddles.clear();
+    ctx->dft_tables.clear();
     if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
     delete ctx;
     return BF_OK;

@@ -16,7 +16,7 @@
 // is therefore exactly two launches (column pass, then fused row pass), each
 // reading and writing every field once.  The per-region k-space phase tables
 // are built once per frequency batch from FP64 arguments.
-#include "bf_internal.h"
+#include "bf_passes.h"
 #include "bf_fftreg.h"
 
 #include <algorithm>
@@ -27,26 +27,6 @@
 #include <cstring>
 
 namespace bf {
-
-// ---------------------------------------------------------------------------
-// descriptors
-// ---------------------------------------------------------------------------
-enum : uint32_t { RF_INV = 1, RF_RTAB = 2, RF_MASK = 4, RF_FWD = 8 };
-enum : uint32_t { CF_FWD = 1, CF_KMID = 2, CF_INV = 4, CF_KLOAD = 8, CF_INSHIFT = 16, CF_OUTSHIFT = 32 };
-enum : uint32_t { DF_FWD = 1, DF_AMAX = 2, DF_EOUT_ASSIGN = 4 };
-enum : int { FD_WHOLE = 1 };  // FieldDesc.pad: column pass stores every row of this field
-constexpr int FD_PAIR_SHIFT = 8;  // FieldDesc.pad >> FD_PAIR_SHIFT: region pair of a cheerleader pair step
-
-// Precision tags: `double` = FP64 storage and arithmetic; `float` = fields stored
-// in FP32 in HBM, all in-register arithmetic (FFTs, phases, boundary updates) in
-// FP64; `f32pure` = FP32 storage and FP32 arithmetic.
-template <typename T> struct Storage { using type = T; };
-template <> struct Storage<f32pure> { using type = float; };
-template <typename T> struct Compute { using type = double; };
-template <> struct Compute<f32pure> { using type = float; };
-#define BF_TYPES(T)                           \
-    using S = typename Storage<T>::type;      \
-    using C = typename Compute<T>::type
 
 // ---------------------------------------------------------------------------
 // small kernels
@@ -119,22 +99,6 @@ __global__ void k_scale_fields(typename Storage<T>::type* base_, const FieldDesc
 // ---------------------------------------------------------------------------
 // row pass
 // ---------------------------------------------------------------------------
-template <typename T>
-struct RowArgs {
-    cplx<typename Storage<T>::type>* base;
-    const FieldDesc* fd;
-    int nf, nx, ny;
-    const cplx<typename Compute<T>::type>* tw;
-    uint32_t flags;
-    const cplx<typename Compute<T>::type>* rtab;
-    const double* X;
-    const double* Y;
-    double R2;
-    const int* active;
-    // rows outside [ylo, yhi) are skipped (not read, not written) when yhi > ylo
-    int ylo, yhi;
-};
-
 template <typename T, int N>
 __global__ void __launch_bounds__(1024) k_rows(RowArgs<T> a) {
     BF_TYPES(T);
@@ -182,31 +146,6 @@ __global__ void __launch_bounds__(1024) k_rows(RowArgs<T> a) {
 // ---------------------------------------------------------------------------
 // column pass
 // ---------------------------------------------------------------------------
-template <typename T>
-struct ColArgs {
-    const cplx<typename Storage<T>::type>* src;
-    cplx<typename Storage<T>::type>* dst;
-    const FieldDesc* fd;
-    int nf, nx, ny;
-    const cplx<typename Compute<T>::type>* tw;
-    uint32_t flags;
-    const cplx<typename Compute<T>::type>* ktab;
-    int tx;  // columns per block
-    const int* active;
-    // Row band: rows outside [ylo, yhi) are known to be zero on input (they are
-    // not loaded) and are not needed on output (not stored), except for the
-    // fields whose descriptor carries FD_WHOLE, stored whole.
-    int ylo, yhi;
-    int kq;  // 0: full k-space tables; else quarter tables of row width kq = nx/2 (dancer propagation)
-    int all_whole;  // every field is stored whole (the band limits the loads only)
-};
-
-template <typename T>
-__device__ __forceinline__ bool in_band(const ColArgs<T>& a, int y) {
-    return (unsigned)(y - a.ylo) < (unsigned)(a.yhi - a.ylo);
-}
-__device__ __forceinline__ bool store_whole(const FieldDesc& d) { return (d.pad & FD_WHOLE) != 0; }
-
 template <typename T, int N>
 __global__ void __launch_bounds__(1024) k_cols(ColArgs<T> a) {
     BF_TYPES(T);
@@ -274,58 +213,6 @@ __global__ void __launch_bounds__(1024) k_cols(ColArgs<T> a) {
 // ---------------------------------------------------------------------------
 // dancer: fused row pass with the boundary update
 // ---------------------------------------------------------------------------
-template <typename T>
-struct DancerRowArgs {
-    cplx<typename Storage<T>::type>* fields;  // [fb][R][2][ny][nx]
-    int R, nx, ny;
-    int rm;  // slot holding the right-moving fields this bounce
-    const cplx<typename Compute<T>::type>* tw;
-    const cplx<typename Compute<T>::type>* rtab;
-    const int* rtab_idx;  // [fb][R], -1: none
-    const zd* coef;       // boundary reflectivities r_b, b = 0..R (r_R = 0 appended)
-    const double* X;
-    const double* Y;
-    double R2;
-    const uint32_t* keep_tab;  // [ny][nx/16] aperture bits of the register path, or null
-    int keep_band;             // band class of keep_tab: no bit outside [keep_band, 15 - keep_band]
-    uint32_t flags;
-    zd* Eout;  // [nslices][ny][nx] per frequency slot, stride eout_fstride
-    size_t eout_fstride;
-    int slice;
-    double* amax;  // [fb]
-    const int* active;
-    int* count;  // [fb] bounce counters
-    // Row band [ylo, yhi): outside it the next bounce's aperture zeroes every
-    // row, so those rows are only needed for Eout at the exit boundary.  The
-    // launcher fills the tile map from the band and its rows per block.
-    int ylo, yhi;
-    int tile0, nband, ntiles;
-};
-
-// Block -> (boundary b, row tile).  Blocks [0, nband (R+1)) cover the row tiles
-// that meet the band at every boundary; the remaining ntiles - nband blocks
-// cover the other row tiles at the exit boundary only (exit_only: Eout is
-// accumulated, nothing is stored because the aperture zeroes those rows).
-template <typename T>
-__device__ __forceinline__ void dancer_block(const DancerRowArgs<T>& a, int i, int& b, int& tile, bool& exit_only) {
-    const int nb = a.nband * (a.R + 1);
-    if (i < nb) {
-        b = i / a.nband;
-        tile = a.tile0 + i % a.nband;
-        exit_only = false;
-    } else {
-        const int j = i - nb;
-        b = a.R;
-        tile = j < a.tile0 ? j : j + a.nband;
-        exit_only = true;
-    }
-}
-
-__device__ __forceinline__ void atomic_max_pos(double* addr, double v) {
-    // non-negative doubles order like their bit patterns
-    atomicMax(reinterpret_cast<unsigned long long*>(addr), (unsigned long long)__double_as_longlong(v));
-}
-
 template <typename T, int N>
 __global__ void __launch_bounds__(1024) k_dancer_rows(DancerRowArgs<T> a) {
     BF_TYPES(T);
@@ -820,6 +707,7 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) k
     dancer_rows_reg_dispatch<float, N, XB>(a);
 }
 
+
 // pointwise bounce update for the unfused propagators (propagator1D, momentum space)
 template <typename T>
 __global__ void k_dancer_update(cplx<typename Storage<T>::type>* fields, int R, size_t K, int rm,
@@ -985,6 +873,8 @@ void Grid::upload(const bf_coords* c, hipStream_t s) {
     bf::upload(Y.p, c->Y, sizeof(double) * ny, s);
     bf::upload(kX.p, c->kX, sizeof(double) * nx, s);
     bf::upload(kY.p, c->kY, sizeof(double) * ny, s);
+    hX.assign(c->X, c->X + nx);
+    hY.assign(c->Y, c->Y + ny);
     hkX.assign(c->kX, c->kX + nx);
     hkY.assign(c->kY, c->kY + ny);
 }
@@ -1003,6 +893,9 @@ const cplx<T>* twiddle_table(bf_ctx* ctx, int n) {
 }
 template const cplx<double>* twiddle_table<double>(bf_ctx*, int);
 template const cplx<float>* twiddle_table<float>(bf_ctx*, int);
+
+// lengths the register transforms do not take
+static bool dft_length(int n) { return !(n >= 16 && (n & (n - 1)) == 0); }
 
 static inline unsigned grid1d(size_t n, int threads, unsigned cap = 2048) {
     size_t b = (n + threads - 1) / threads;
@@ -1028,6 +921,7 @@ static void dispatch_n(int n, A&&... args) {
 
 static bool use_reg_fft() { return !opts().fft_lds; }
 
+
 template <typename T, int N>
 struct RowLaunch {
     static void run(const RowArgs<T>& a, hipStream_t s) {
@@ -1042,6 +936,12 @@ struct RowLaunch {
                 hipLaunchKernelGGL((k_rows_reg<T, N>), dim3((unsigned)((nlines + lpb - 1) / lpb)), dim3(lpb * C::TT),
                                    smem, s, a);
                 BF_CHECK_LAUNCH();
+                return;
+            }
+        }
+        if constexpr (N < 16 && std::is_same<typename Compute<T>::type, double>::value) {
+            if (use_reg_fft() && a.dft.tab) {
+                launch_rows_dft<T>(a, s);
                 return;
             }
         }
@@ -1107,6 +1007,12 @@ struct ColLaunch {
                 return;
             }
         }
+        if constexpr (N < 16 && std::is_same<typename Compute<T>::type, double>::value) {
+            if (use_reg_fft() && a.dft.tab) {
+                launch_cols_dft<T>(a, s);
+                return;
+            }
+        }
         const int TPL = LineCfg<N>::TPL;
         const int n = N >= 16 ? N : a.ny;
         int tx = tx_req > 0 ? tx_req : (int)(128 / sizeof(cplx<typename Storage<T>::type>));
@@ -1119,19 +1025,6 @@ struct ColLaunch {
         BF_CHECK_LAUNCH();
     }
 };
-
-template <typename T>
-static unsigned dancer_tiles(DancerRowArgs<T>& a, int rows) {
-    a.ntiles = (a.ny + rows - 1) / rows;
-    if (a.yhi > a.ylo) {
-        a.tile0 = a.ylo / rows;
-        a.nband = (a.yhi + rows - 1) / rows - a.tile0;
-    } else {
-        a.tile0 = 0;
-        a.nband = 0;
-    }
-    return (unsigned)(a.nband * (a.R + 1) + (a.ntiles - a.nband));
-}
 
 template <typename T, int N>
 struct DancerRowLaunch {
@@ -1168,6 +1061,12 @@ struct DancerRowLaunch {
                 return;
             }
         }
+        if constexpr (N < 16 && std::is_same<typename Compute<T>::type, double>::value) {
+            if (use_reg_fft() && a.dft.tab) {
+                launch_dancer_rows_dft<T>(a, fb, s);
+                return;
+            }
+        }
         const int TPL = LineCfg<N>::TPL;
         const int n = N >= 16 ? N : a.nx;
         int rows = rows_req > 0 ? rows_req : std::max(1, 128 / TPL);
@@ -1185,6 +1084,23 @@ struct DancerRowLaunch {
 // ---------------------------------------------------------------------------
 // Julia: k0 = 2*pi/lambda*sqrt(eps)
 static inline zd k0_of(zd eps, double lambda) { return rmul((2.0 * M_PI) / lambda, csqrt_j(eps)); }
+
+// Entries u of one axis with axis[u]^2 + min(other^2) < diskR^2 (a relative margin of
+// 1e-9 keeps every one the device mask could keep): [lo, hi), or [0, 0) when none.
+static void aperture_range(const std::vector<double>& axis, const std::vector<double>& other, double diskR, int& lo,
+                           int& hi) {
+    double min2 = INFINITY;
+    for (double v : other) min2 = std::min(min2, v * v);
+    const double lim = diskR * diskR * (1.0 + 1e-9);
+    lo = (int)axis.size();
+    hi = 0;
+    for (int u = 0; u < (int)axis.size(); u++)
+        if (axis[u] * axis[u] + min2 < lim) {
+            lo = std::min(lo, u);
+            hi = u + 1;
+        }
+    if (lo >= hi) lo = hi = 0;
+}
 
 // One propagation region at one frequency: what a prop() call needs.
 struct RegionParams {
@@ -1213,11 +1129,27 @@ struct PropEngine {
     bool quarter = false;
     // aperture row band [blo, bhi) of propagate() (bhi <= blo: every row)
     int blo = 0, bhi = 0;
+    // matrix-core transforms of the lines that are no power of two (FP64 arithmetic)
+    std::shared_ptr<DevBuf> dftx, dfty;
+    int dft_xlo = 0;  // smallest folded x index inside the aperture
 
     PropEngine(bf_ctx* c, const Grid* gr, int k, double diskR, const zd* surf)
         : ctx(c), g(gr), kind(k), R2(diskR * diskR), surfaces(surf) {
         twx = twiddle_table<C>(ctx, g->nx);
         twy = twiddle_table<C>(ctx, g->ny);
+        if (std::is_same<C, double>::value && use_reg_fft()) {
+            if (dft_length(g->nx)) dftx = dft_table(ctx, g->nx);
+            if (dft_length(g->ny)) dfty = dft_table(ctx, g->ny);
+            int lo, hi;
+            aperture_range(g->hX, g->hY, diskR, lo, hi);
+            dft_xlo = hi > lo ? dft_fold_lo(g->nx, lo, hi) : g->nx / 2;
+        }
+    }
+    DftArgs dft_x() const {
+        DftArgs d;
+        d.tab = dftx ? dftx->template as<double2>() : nullptr;
+        d.lo = dft_xlo;
+        return d;
     }
 
     // Build the k-space and real-space tables for a list of regions.  With
@@ -1300,6 +1232,7 @@ struct PropEngine {
         a.base = base; a.fd = fd; a.nf = nf; a.nx = g->nx; a.ny = g->ny; a.tw = twx; a.flags = flags;
         a.rtab = rtab.as<cplx<C>>(); a.X = g->X.as<double>(); a.Y = g->Y.as<double>(); a.R2 = R2; a.active = active;
         a.ylo = ylo; a.yhi = yhi;
+        a.dft = dft_x();
         dispatch_n<RowLaunch, T>(g->nx, a, ctx->stream);
     }
     // ylo/yhi: row band (yhi < 0: all rows); all_whole: store every row of every field
@@ -1311,6 +1244,7 @@ struct PropEngine {
         a.kq = quarter ? g->nx / 2 : 0;
         a.all_whole = all_whole ? 1 : 0;
         a.ylo = ylo; a.yhi = yhi < 0 ? g->ny : yhi;
+        if (dfty) a.dft.tab = dfty->template as<double2>();
         dispatch_n<ColLaunch, T>(g->ny, a, col_tx, ctx->stream);
     }
 
@@ -1478,22 +1412,6 @@ static bool quarter_tables_ok(const bf_coords* co, int kind) {
            (n & (n - 1)) == 0 && mirrored(co->kX, co->nx) && mirrored(co->kY, co->ny);
 }
 
-// Rows y with Y[y]^2 + min_x X[x]^2 < diskR^2 (a relative margin of 1e-9 keeps
-// every row the device mask could keep): [lo, hi), or [0, 0) when none.
-static void aperture_band(const bf_coords* co, double diskR, int& lo, int& hi) {
-    double minx2 = INFINITY;
-    for (int x = 0; x < co->nx; x++) minx2 = std::min(minx2, co->X[x] * co->X[x]);
-    const double lim = diskR * diskR * (1.0 + 1e-9);
-    lo = co->ny;
-    hi = 0;
-    for (int y = 0; y < co->ny; y++)
-        if (co->Y[y] * co->Y[y] + minx2 < lim) {
-            lo = std::min(lo, y);
-            hi = y + 1;
-        }
-    if (lo >= hi) lo = hi = 0;
-}
-
 template <typename T>
 struct DancerPlan : DancerPlanBase {
     BF_TYPES(T);
@@ -1603,7 +1521,7 @@ struct DancerPlan : DancerPlanBase {
         band_lo = 0;
         band_hi = g.ny;
         if (opt.band && amin == 0.0 && (kind == BF_PROP_PROPAGATOR || kind == BF_PROP_NOTILTS))
-            aperture_band(co, diskR, band_lo, band_hi);
+            aperture_range(g.hY, g.hX, diskR, band_lo, band_hi);
         const bool qtab = quarter_tables_ok<T>(co, kind);
         // Frequency batch: what one bounce of a batch touches (the band rows of every
         // field, plus one k-space table per distinct (eps, dz)) is kept near
@@ -1727,6 +1645,7 @@ struct DancerPlan : DancerPlanBase {
             a.count = count.as<int>() + f0;
             a.ylo = band_lo;
             a.yhi = band_hi;
+            a.dft = pe->dft_x();
             tmark(n, 0, 0);
             dispatch_n<DancerRowLaunch, T>(g.nx, a, nb, opt.rows, s);
             tmark(n, 0, 1);
@@ -2083,24 +2002,6 @@ __global__ void k_ch_pair(cplx<typename Storage<T>::type>* F, int Nd, size_t K, 
 // of their next propagation zeroes them.  With xout the kernel also starts
 // that next propagation: the updated rows are masked by the aperture and
 // transformed along x (the masked row FFT of k_rows_reg) before they are stored.
-template <typename T>
-struct ChPairArgs {
-    cplx<typename Storage<T>::type>* F;  // [fb][Nd][K]
-    // entry e (one frequency of one region pair (i, i+1)): fd[2e] field i,
-    // fd[2e+1] field i+1; i = fd[2e].pad >> FD_PAIR_SHIFT
-    const FieldDesc* fd;
-    int ny, rows;
-    const cplx<typename Compute<T>::type>* tw;
-    const cplx<typename Compute<T>::type>* rtab;  // null: no tilt/surface tables
-    const zd* coef;  // [i][4]: rl, tr, rr, tl of boundary i
-    const int* active;
-    int ylo, yhi;  // rows processed
-    int xout;      // store the masked row transform of the updated fields
-    const double* X;
-    const double* Y;
-    double R2;  // aperture radius squared
-};
-
 template <typename T, int N>
 __global__ void __launch_bounds__(512) k_ch_pair_rows(ChPairArgs<T> a) {
     BF_TYPES(T);
@@ -2165,10 +2066,11 @@ __global__ void __launch_bounds__(512) k_ch_pair_rows(ChPairArgs<T> a) {
         if (ok) line[TT * m] = ccast<S>(v[m]);
 }
 
+
 template <typename T, int N>
 struct ChPairLaunch {
     // nb: entries (region pair x frequency) in a.fd
-    static void run(ChPairArgs<T> a, int nb, hipStream_t s) {
+    static void run(ChPairArgs<T> a, int nx, int nb, hipStream_t s) {
         if constexpr (N >= 16) {
             using C = RegE<T, N>;
             a.rows = std::max(1, 128 / C::TT);
@@ -2177,6 +2079,8 @@ struct ChPairLaunch {
             hipLaunchKernelGGL((k_ch_pair_rows<T, N>), dim3((a.yhi - a.ylo + a.rows - 1) / a.rows, nb),
                                dim3(2 * a.rows * C::TT), smem, s, a);
             BF_CHECK_LAUNCH();
+        } else if constexpr (std::is_same<typename Compute<T>::type, double>::value) {
+            launch_ch_pair_dft<T>(a, nx, nb, s);
         } else {
             throw Error(BF_ERR_UNSUPPORTED, "fused cheerleader rows need a power-of-two grid of at least 16");
         }
@@ -2263,11 +2167,12 @@ void cheerleader_run(bf_ctx* ctx, const bf_setup* st, const bf_coords* co, doubl
     {
         // every propagation starts by masking: its masked row FFT and column pass
         // need only the aperture's row band (register path; option band=0 disables)
-        auto pow2 = [](int n) { return n >= 16 && n <= 1024 && (n & (n - 1)) == 0; };
-        if (opts().band && use_reg_fft() && pow2(g.nx) && pow2(g.ny) &&
+        // (the matrix-core passes of the other lengths, FP64 arithmetic, do the same)
+        auto fast = [&](int n) { return !dft_length(n) || std::is_same<C, double>::value; };
+        if (opts().band && use_reg_fft() && fast(g.nx) && fast(g.ny) &&
             (kind == BF_PROP_PROPAGATOR || kind == BF_PROP_NOTILTS))
-            aperture_band(co, diskR, pe.blo, pe.bhi);
-        fuse_pair = opts().chfuse && use_reg_fft() && pow2(g.nx) &&
+            aperture_range(g.hY, g.hX, diskR, pe.blo, pe.bhi);
+        fuse_pair = opts().chfuse && use_reg_fft() && fast(g.nx) &&
                     (kind == BF_PROP_PROPAGATOR || kind == BF_PROP_NOTILTS);
     }
     // The pair steps update the interior fields F[1..Nd-2] only; each is masked
@@ -2415,7 +2320,8 @@ void cheerleader_run(bf_ctx* ctx, const bf_setup* st, const bf_coords* co, doubl
             pa.active = A;
             pa.xout = pair_xform ? 1 : 0;
             pa.X = g.X.as<double>(); pa.Y = g.Y.as<double>(); pa.R2 = pe.R2;
-            dispatch_n<ChPairLaunch, T>(g.nx, pa, entries, s);
+            pa.dft = pe.dft_x();
+            dispatch_n<ChPairLaunch, T>(g.nx, pa, g.nx, entries, s);
         };
         if (wave) {
             // per time: masked row FFT of the fields in real space (r1), column pass

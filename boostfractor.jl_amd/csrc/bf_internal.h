@@ -131,6 +131,8 @@ struct bf_ctx {
     std::string err;
     // twiddle tables keyed by (n, bytes per real)
     std::map<std::pair<int, int>, bf::DevBuf> twiddles;
+    // matrices of the matrix-core line transforms, most recently used last
+    std::vector<std::pair<int, std::shared_ptr<bf::DevBuf>>> dft_tables;
     bool timing = false;
     std::map<std::string, bf_kernel_timer> timers;
     // grow-only device buffers reused by consecutive calls on this context
@@ -272,7 +274,7 @@ void clear_timers(bf_ctx* ctx);
 struct Grid {
     int nx = 0, ny = 0;
     DevBuf X, Y, kX, kY;  // double
-    std::vector<double> hkX, hkY;  // host copies of kX, kY
+    std::vector<double> hX, hY, hkX, hkY;  // host copies
     void upload(const bf_coords* c, hipStream_t s);
     size_t K() const { return (size_t)nx * ny; }
 };
