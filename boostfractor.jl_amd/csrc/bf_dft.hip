@@ -9,32 +9,114 @@ namespace bf {
 // ---------------------------------------------------------------------------
 // matrix-core versions of the passes (bf_dftmm.h): FP64 arithmetic, any line
 // length up to 1023 that the register transforms do not take.  A block of one
-// wave per 16 output indices holds 8 lines.  What bounds them: at 101^2 a bounce
-// of 16 frequencies moves 44 MB (the band rows of 224 fields, in and out) and
-// issues 2.9e5 MFMAs, 3 us of HBM and 7 us of matrix-core time; the direct sum in
-// LDS they replace spent 650 us per bounce on it (LDS reads and 8 n^2 FMAs a line).
+// wave per 16 output indices holds 8 lines.  What bounds them: a bounce of 16
+// frequencies and 3 disks at 101^2 moves 44 MB (the band rows of 224 fields, in
+// and out) and issues 3.2e5 MFMAs, 8 us of HBM and 9 us of matrix-core time; the
+// column pass takes 27 us and the row pass 19 us, in chains of dependent loads
+// (kernel arguments, descriptor, lines, output) with 4 waves per SIMD.  The
+// direct sums in LDS that they replace took 458 and 193 us (8 n^2 FMAs a line and
+// an LDS read for each).  Loads predicated by an out-of-range buffer offset
+// instead of branches, the sine and the cosine product of a shared tile in waves
+// of their own, and the tables' loads issued before the first wait brought them
+// from 38 and 25 us.
 // ---------------------------------------------------------------------------
-template <typename T, int TPW>
+// FL != 0: the flags are fixed at compile time (the solvers' FWD|KMID|INV, no shifts)
+template <typename T, int TPW, uint32_t FL>
 __global__ void __launch_bounds__(1024) k_cols_dft(ColArgs<T> a) {
     using S = typename Storage<T>::type;
-    extern __shared__ unsigned char smem_raw[];
-    const int n = a.ny, nx = a.nx, H = n >> 1, ld = dft_ld(n);
-    double* E = reinterpret_cast<double*>(smem_raw);
-    double* O = E + dft_rows(n, 0) * DFT_LDP;
-    double* part = O + dft_rows(n, 0) * DFT_LDP;
+    extern __shared__ double2 dft_smem[];
+    const int n = a.ny, nx = a.nx, H = n >> 1;
+    double2* P = dft_smem;
+    double2* part = P + dft_rows(n, 0) * DFT_LDP;
     const FieldDesc d = a.fd[blockIdx.y];
-    if (a.active && !a.active[d.group]) return;  // uniform over the block
+    const bool idle = a.active && !a.active[d.group];  // uniform over the block
+    const int W = blockDim.x >> 6, lane = threadIdx.x & 63;
     const int x0 = blockIdx.x * DFT_LINES;
+    constexpr uint32_t PROP = CF_FWD | CF_KMID | CF_INV, SZ = sizeof(cplx<S>);
+    const uint32_t fl = FL ? FL : a.flags;
+    dbl4 e[TPW], o[TPW];
+    if constexpr (FL == PROP) {
+        // A resource over the band rows answers the others with zero, as one over the
+        // k-space table answers bins without a mirror: no branch on either
+        const bool whole = store_whole(d) || a.all_whole;
+        const int band = dft_fold_lo(n, a.ylo, a.yhi), base = band & ~3, rows = dft_rows(n, base);
+        const uint32_t rowb = (uint32_t)nx * SZ, bandb = (uint32_t)(a.yhi - a.ylo) * rowb;
+        const auto rs = buf_rsrc(a.src + d.off + (size_t)a.ylo * nx, bandb);
+        const uint32_t KT = (uint32_t)n * (uint32_t)nx * (uint32_t)sizeof(zd), krow = (uint32_t)nx * (uint32_t)sizeof(zd);
+        const auto rk = buf_rsrc(a.ktab + (size_t)d.ktab * n * nx, KT);
+        int mt = dft_tiles(n, 0);
+        const DftShare s1(mt, a.dft.smax);
+        // The field's and the phase table's loads go out together, before anything waits:
+        // a dependent load costs ~1 us here, more than the products of a stage.
+        const int c = threadIdx.x & 7, r0 = threadIdx.x >> 3, rstep = blockDim.x >> 3;
+        const uint32_t cb = (uint32_t)(x0 + c) * SZ - (uint32_t)a.ylo * rowb;
+        auto point = [&](int r, cplx<S>& x, cplx<S>& m) {
+            const int j = base + r;
+            const bool in = x0 + c < nx && j <= H;
+            x = buf_load<S>(rs, in ? cb + (uint32_t)j * rowb : BUF_OOB);
+            m = buf_load<S>(rs, in && j > 0 && 2 * j < n ? cb + (uint32_t)(n - j) * rowb : BUF_OOB);
+        };
+        cplx<S> x, m;
+        point(r0, x, m);
+        zd pv[TPW][2], pm[TPW][2];
+#pragma unroll
+        for (int q = 0; q < TPW; q++)
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                const int mx = x0 + 4 * h + (lane >> 4), k = 16 * (s1.first + q * W) + (lane & 15);
+                const bool in = mx < nx && k <= H && s1.s == 0;
+                const uint32_t kb = (uint32_t)mx * (uint32_t)sizeof(zd);
+                pv[q][h] = buf_load<double>(rk, in ? kb + (uint32_t)k * krow : BUF_OOB);
+                pm[q][h] = buf_load<double>(rk, in && k > 0 && 2 * k < n ? kb + (uint32_t)(n - k) * krow : BUF_OOB);
+            }
+        if (idle) return;
+        for (int r = r0; r < rows; r += rstep) {
+            if (r != r0) point(r, x, m);
+            dft_fold<false>(P, r, c, ccast<double>(x), ccast<double>(m));
+        }
+        dft_stage<TPW>(P, part, n, base, 0, mt, s1, a.dft.tab, e, o);
+        // k-space phase of bin k and of its mirror, folded for the inverse
+        if (s1.own(mt))
+#pragma unroll
+            for (int q = 0; q < TPW; q++) {
+                const int k = 16 * (s1.first + q * W) + (lane & 15);
+                if (s1.first + q * W < mt && k < dft_rows(n, 0))
+#pragma unroll
+                    for (int h = 0; h < 2; h++)
+                        dft_fold<true>(P, k, 4 * h + (lane >> 4), cmul(dft_out(e[q], o[q], h), pv[q][h]),
+                                       cmul(dft_mirror(e[q], o[q], h), pm[q][h]));
+            }
+        const int b0 = whole ? 0 : band;
+        mt = dft_tiles(n, b0);
+        const DftShare s2(mt, a.dft.smax);
+        dft_stage<TPW>(P, part, n, 0, b0, mt, s2, a.dft.tab, e, o);
+        if (!s2.own(mt)) return;
+        // band rows, or every row of a field stored whole
+        const int s0 = whole ? 0 : a.ylo;
+        const auto rd = buf_rsrc(a.dst + d.off + (size_t)s0 * nx, whole ? (uint32_t)n * rowb : bandb);
+#pragma unroll
+        for (int q = 0; q < TPW; q++) {
+            const int j = b0 + 16 * (s2.first + q * W) + (lane & 15);
+            if (s2.first + q * W >= mt) continue;
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                const int mx = x0 + 4 * h + (lane >> 4);
+                const bool in = mx < nx && j <= H;
+                const uint32_t cb = (uint32_t)mx * SZ - (uint32_t)s0 * rowb;
+                buf_store<S>(rd, in ? cb + (uint32_t)j * rowb : BUF_OOB, ccast<S>(dft_out(e[q], o[q], h)));
+                buf_store<S>(rd, in && j > 0 && 2 * j < n ? cb + (uint32_t)(n - j) * rowb : BUF_OOB,
+                             ccast<S>(dft_mirror(e[q], o[q], h)));
+            }
+        }
+        return;
+    }
+    if (idle) return;
+    // one transform, or shifted loads and stores (momentum space): every row
     const int hx = nx / 2, hy = n / 2;
-    const uint32_t fl = a.flags;
     const cplx<S>* src = a.src + d.off;
     cplx<S>* dst = a.dst + d.off;
     const zd* kt = d.ktab >= 0 ? a.ktab + (size_t)d.ktab * n * nx : nullptr;
-    const bool whole = store_whole(d) || a.all_whole || (fl & (CF_INSHIFT | CF_OUTSHIFT));
-    const int band = (fl & (CF_INSHIFT | CF_OUTSHIFT)) ? 0 : dft_fold_lo(n, a.ylo, a.yhi);
     const bool fwd = (fl & CF_FWD) != 0, two = fwd && (fl & CF_INV);
-    // fold the input lines (rows outside the band are zero)
-    const int base = band & ~3, rows = dft_rows(n, base);
     auto load = [&](int y, int mx) -> zd {
         int sx = mx, sy = y;
         if (fl & CF_INSHIFT) {  // ifftshift on load
@@ -42,33 +124,30 @@ __global__ void __launch_bounds__(1024) k_cols_dft(ColArgs<T> a) {
             sy = (y + hy) % n;
         }
         if (!in_band(a, sy)) return cmk<double>(0, 0);
-        const size_t o = (size_t)sy * nx + sx;
-        zd v = ccast<double>(src[o]);
-        if ((fl & CF_KLOAD) && kt) v = cmul(v, ccast<double>(kt[o]));
+        const size_t p = (size_t)sy * nx + sx;
+        zd v = ccast<double>(src[p]);
+        if ((fl & CF_KLOAD) && kt) v = cmul(v, ccast<double>(kt[p]));
         return v;
     };
-    for (int q = threadIdx.x; q < rows * DFT_LINES; q += blockDim.x) {
-        const int c = q & (DFT_LINES - 1), r = q / DFT_LINES, j = base + r, mx = x0 + c;
-        const bool ok = mx < nx && j <= H, pr = ok && dft_paired(n, j);
+    for (int q = threadIdx.x; q < dft_rows(n, 0) * DFT_LINES; q += blockDim.x) {
+        const int c = q & (DFT_LINES - 1), j = q / DFT_LINES, mx = x0 + c;
+        const bool ok = mx < nx && j <= H;
         const zd x = ok ? load(j, mx) : cmk<double>(0, 0);
-        const zd m = pr ? load(n - j, mx) : cmk<double>(0, 0);
+        const zd m = ok && dft_paired(n, j) ? load(n - j, mx) : cmk<double>(0, 0);
         if (fwd)
-            dft_fold<false>(E, O, r, c, pr, x, m);
+            dft_fold<false>(P, j, c, x, m);
         else
-            dft_fold<true>(E, O, r, c, pr, x, m);
+            dft_fold<true>(P, j, c, x, m);
     }
-    const int W = blockDim.x >> 6, lane = threadIdx.x & 63;
-    dbl4 e[TPW], o[TPW];
-    int tile0, mt = dft_tiles(n, 0), b0 = 0;
-    bool own;
+    const int mt = dft_tiles(n, 0);
+    const DftShare sh(mt, a.dft.smax);
+    dft_stage<TPW>(P, part, n, 0, 0, mt, sh, a.dft.tab, e, o);
     if (two) {
-        own = dft_stage<TPW>(E, O, part, n, base, 0, mt, a.dft.smax, a.dft.tab, ld, e, o, tile0);
-        // k-space phase of bin k and of its mirror, folded for the inverse
-        if (own)
+        if (sh.own(mt))
 #pragma unroll
             for (int q = 0; q < TPW; q++) {
-                const int k = 16 * (tile0 + q * W) + (lane & 15);
-                if (tile0 + q * W < mt && k < dft_rows(n, 0)) {
+                const int k = 16 * (sh.first + q * W) + (lane & 15);
+                if (sh.first + q * W < mt && k < dft_rows(n, 0)) {
                     const bool pr = dft_paired(n, k);
 #pragma unroll
                     for (int h = 0; h < 2; h++) {
@@ -80,19 +159,14 @@ __global__ void __launch_bounds__(1024) k_cols_dft(ColArgs<T> a) {
                             v = cmul(v, ccast<double>(kt[(size_t)k * nx + mx]));
                             if (pr) m = cmul(m, ccast<double>(kt[(size_t)(n - k) * nx + mx]));
                         }
-                        dft_fold<true>(E, O, k, c, pr, v, m);
+                        dft_fold<true>(P, k, c, v, m);
                     }
                 }
             }
-        b0 = whole ? 0 : band;
-        mt = dft_tiles(n, b0);
-        own = dft_stage<TPW>(E, O, part, n, 0, b0, mt, a.dft.smax, a.dft.tab, ld, e, o, tile0);
-    } else {
-        b0 = whole || fwd ? 0 : band;
-        mt = dft_tiles(n, b0);
-        own = dft_stage<TPW>(E, O, part, n, base, b0, mt, a.dft.smax, a.dft.tab, ld, e, o, tile0);
+        dft_stage<TPW>(P, part, n, 0, 0, mt, sh, a.dft.tab, e, o);
     }
-    if (!own) return;
+    if (!sh.own(mt)) return;
+    const bool whole = store_whole(d) || a.all_whole;
     auto store = [&](int y, int mx, zd v) {
         int dx = mx, dy = y;
         if (fl & CF_OUTSHIFT) {  // fftshift on store
@@ -103,8 +177,8 @@ __global__ void __launch_bounds__(1024) k_cols_dft(ColArgs<T> a) {
     };
 #pragma unroll
     for (int q = 0; q < TPW; q++) {
-        const int j = b0 + 16 * (tile0 + q * W) + (lane & 15);
-        if (tile0 + q * W >= mt || j > H) continue;
+        const int j = 16 * (sh.first + q * W) + (lane & 15);
+        if (sh.first + q * W >= mt || j > H) continue;
 #pragma unroll
         for (int h = 0; h < 2; h++) {
             const int mx = x0 + 4 * h + (lane >> 4);
@@ -115,18 +189,32 @@ __global__ void __launch_bounds__(1024) k_cols_dft(ColArgs<T> a) {
     }
 }
 
+// Loads and folds line `c` of the block (one wave per line, lanes along it) from
+// its first element p; null: a zero line.  map(x, v): value of element x.
+template <bool INV, typename S, typename F>
+__device__ __forceinline__ void dft_load_line(double2* P, int n, int base, int c, const cplx<S>* p, F map) {
+    const int lane = threadIdx.x & 63, rows = dft_rows(n, base);
+    const auto r = buf_rsrc(p, p ? (uint32_t)n * (uint32_t)sizeof(cplx<S>) : 0u);
+    for (int q = lane; q < rows; q += 64) {
+        const int j = base + q;
+        const bool in = j <= n >> 1, pr = in && j > 0 && 2 * j < n;
+        const cplx<S> x = buf_load<S>(r, in ? (uint32_t)j * (uint32_t)sizeof(cplx<S>) : BUF_OOB);
+        const cplx<S> m = buf_load<S>(r, pr ? (uint32_t)(n - j) * (uint32_t)sizeof(cplx<S>) : BUF_OOB);
+        dft_fold<INV>(P, q, c, map(in ? j : 0, ccast<double>(x)), map(pr ? n - j : 0, ccast<double>(m)));
+    }
+}
+
 template <typename T, int TPW>
 __global__ void __launch_bounds__(1024) k_rows_dft(RowArgs<T> a) {
     using S = typename Storage<T>::type;
-    extern __shared__ unsigned char smem_raw[];
-    const int n = a.nx, H = n >> 1, ld = dft_ld(n);
-    double* E = reinterpret_cast<double*>(smem_raw);
-    double* O = E + dft_rows(n, 0) * DFT_LDP;
-    double* part = O + dft_rows(n, 0) * DFT_LDP;
+    extern __shared__ double2 dft_smem[];
+    const int n = a.nx, H = n >> 1;
+    double2* P = dft_smem;
+    double2* part = P + dft_rows(n, 0) * DFT_LDP;
     // the grid covers the rows [ylo, yhi) of every field (all rows when yhi <= ylo)
     const bool yband = a.yhi > a.ylo;
     const int nr = yband ? a.yhi - a.ylo : a.ny, y0 = yband ? a.ylo : 0;
-    const long nlines = (long)a.nf * nr, line0 = (long)blockIdx.x * DFT_LINES;
+    const int nlines = a.nf * nr, line0 = blockIdx.x * DFT_LINES;
     const uint32_t fl = a.flags;
     const bool inv = (fl & RF_INV) != 0, two = inv && (fl & RF_FWD), mask = (fl & RF_MASK) != 0;
     const size_t K = (size_t)n * a.ny;
@@ -136,73 +224,62 @@ __global__ void __launch_bounds__(1024) k_rows_dft(RowArgs<T> a) {
         if (mask && !in_aperture(a.X[x], a.Y[y], a.R2)) v = cmk<double>(0, 0);
         return v;
     };
-    const int a0 = !inv && mask ? a.dft.lo & ~3 : 0, rows = dft_rows(n, a0);
-    for (int q = threadIdx.x; q < rows * DFT_LINES; q += blockDim.x) {
-        const int c = q / rows, r = q - c * rows, j = a0 + r;
-        const long l = line0 + c;
-        bool ok = l < nlines && j <= H;
-        zd x = cmk<double>(0, 0), m = x;
-        const bool pr = dft_paired(n, j);
-        if (ok) {
-            const FieldDesc d = a.fd[l / nr];
-            const int y = y0 + (int)(l % nr);
-            if (!a.active || a.active[d.group]) {
-                const cplx<S>* row = a.base + d.off + (size_t)y * n;
-                x = ccast<double>(row[j]);
-                if (pr) m = ccast<double>(row[n - j]);
-                if (!inv) {
-                    x = middle(d, y, j, x);
-                    if (pr) m = middle(d, y, n - j, m);
-                }
-            }
-        }
+    const int a0 = !inv && mask ? a.dft.lo & ~3 : 0;
+    const int W = blockDim.x >> 6, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    for (int c = wave; c < DFT_LINES; c += W) {
+        const int l = line0 + c;
+        const FieldDesc d = a.fd[l < nlines ? l / nr : 0];
+        const int y = y0 + (l < nlines ? l % nr : 0);
+        const bool ok = l < nlines && (!a.active || a.active[d.group]);
+        const cplx<S>* p = ok ? a.base + d.off + (size_t)y * n : nullptr;
         if (inv)
-            dft_fold<true>(E, O, r, c, pr && ok, x, m);
+            dft_load_line<true>(P, n, a0, c, p, [](int, zd v) { return v; });
         else
-            dft_fold<false>(E, O, r, c, pr && ok, x, m);
+            dft_load_line<false>(P, n, a0, c, p, [&](int x, zd v) { return middle(d, y, x, v); });
     }
-    const int W = blockDim.x >> 6, lane = threadIdx.x & 63;
     // this lane's two lines
     FieldDesc d[2];
     int y[2];
     bool ok[2];
 #pragma unroll
     for (int h = 0; h < 2; h++) {
-        const long l = line0 + 4 * h + (lane >> 4);
+        const int l = line0 + 4 * h + (lane >> 4);
         ok[h] = l < nlines;
         d[h] = a.fd[ok[h] ? l / nr : 0];
-        y[h] = y0 + (int)(ok[h] ? l % nr : 0);
+        y[h] = y0 + (ok[h] ? l % nr : 0);
         if (a.active && !a.active[d[h].group]) ok[h] = false;
     }
     dbl4 e[TPW], o[TPW];
-    int tile0, b0 = two && mask ? a.dft.lo : 0, mt = dft_tiles(n, b0);
-    bool own = dft_stage<TPW>(E, O, part, n, a0, b0, mt, a.dft.smax, a.dft.tab, ld, e, o, tile0);
+    int b0 = two && mask ? a.dft.lo : 0, mt = dft_tiles(n, b0);
+    DftShare sh(mt, a.dft.smax);
+    dft_stage<TPW>(P, part, n, a0, b0, mt, sh, a.dft.tab, e, o);
     if (two) {
         const int a2 = b0 & ~3;  // the mask zeroes the folded indices below b0
-        if (own)
+        if (sh.own(mt))
 #pragma unroll
             for (int q = 0; q < TPW; q++) {
-                const int j = b0 + 16 * (tile0 + q * W) + (lane & 15);
-                if (tile0 + q * W >= mt || j > H) continue;
+                const int j = b0 + 16 * (sh.first + q * W) + (lane & 15);
+                if (sh.first + q * W >= mt || j > H) continue;
                 const bool pr = dft_paired(n, j);
 #pragma unroll
                 for (int h = 0; h < 2; h++) {
                     const zd v = middle(d[h], y[h], j, dft_out(e[q], o[q], h));
                     const zd m = pr ? middle(d[h], y[h], n - j, dft_mirror(e[q], o[q], h)) : cmk<double>(0, 0);
-                    dft_fold<false>(E, O, j - a2, 4 * h + (lane >> 4), pr, v, m);
+                    dft_fold<false>(P, j - a2, 4 * h + (lane >> 4), v, m);
                 }
             }
-        dft_zero_rows(E, O, 0, b0 - a2);
-        dft_zero_rows(E, O, H + 1 - a2, dft_rows(n, a2));
+        dft_zero_rows(P, 0, b0 - a2);
+        dft_zero_rows(P, H + 1 - a2, dft_rows(n, a2));
         b0 = 0;
         mt = dft_tiles(n, 0);
-        own = dft_stage<TPW>(E, O, part, n, a2, 0, mt, a.dft.smax, a.dft.tab, ld, e, o, tile0);
+        sh = DftShare(mt, a.dft.smax);
+        dft_stage<TPW>(P, part, n, a2, 0, mt, sh, a.dft.tab, e, o);
     }
-    if (!own) return;
+    if (!sh.own(mt)) return;
 #pragma unroll
     for (int q = 0; q < TPW; q++) {
-        const int j = b0 + 16 * (tile0 + q * W) + (lane & 15);
-        if (tile0 + q * W >= mt || j > H) continue;
+        const int j = b0 + 16 * (sh.first + q * W) + (lane & 15);
+        if (sh.first + q * W >= mt || j > H) continue;
 #pragma unroll
         for (int h = 0; h < 2; h++) {
             if (!ok[h]) continue;
@@ -221,48 +298,53 @@ __global__ void __launch_bounds__(1024) k_rows_dft(RowArgs<T> a) {
 template <typename T, int TPW>
 __global__ void __launch_bounds__(1024) k_dancer_rows_dft(DancerRowArgs<T> a) {
     using S = typename Storage<T>::type;
-    extern __shared__ unsigned char smem_raw[];
+    extern __shared__ double2 dft_smem[];
     __shared__ double red[16];
-    const int n = a.nx, H = n >> 1, ld = dft_ld(n);
-    double* E = reinterpret_cast<double*>(smem_raw);
-    double* O = E + dft_rows(n, 0) * DFT_LDP;
-    double* part = O + dft_rows(n, 0) * DFT_LDP;
+    const int n = a.nx, H = n >> 1;
+    double2* P = dft_smem;
+    double2* part = P + dft_rows(n, 0) * DFT_LDP;
     const int f = blockIdx.y;
     int b, tile;
     bool exit_only;
     dancer_block(a, blockIdx.x, b, tile, exit_only);
-    if (a.active && !a.active[f]) return;  // uniform over the block
-    if (a.count && blockIdx.x == 0 && threadIdx.x == 0) a.count[f] += 1;
+    const bool idle = a.active && !a.active[f];  // uniform over the block
     const size_t K = (size_t)n * a.ny;
     const int y0 = tile * 4;
     const bool hasA = b > 0, hasB = b < a.R;
     cplx<S>* FA = a.fields + (((size_t)f * a.R + (hasA ? b - 1 : 0)) * 2 + a.rm) * K;
     cplx<S>* FB = a.fields + (((size_t)f * a.R + (hasB ? b : 0)) * 2 + (1 - a.rm)) * K;
-    const int rows = dft_rows(n, 0);
-    for (int q = threadIdx.x; q < rows * DFT_LINES; q += blockDim.x) {
-        const int c = q / rows, j = q - c * rows, y = y0 + (c & 3);
-        const bool ok = (c < 4 ? hasA : hasB) && y < a.ny && j <= H, pr = dft_paired(n, j);
-        const cplx<S>* row = (c < 4 ? FA : FB) + (size_t)y * n;
-        const zd x = ok ? ccast<double>(row[j]) : cmk<double>(0, 0);
-        const zd m = ok && pr ? ccast<double>(row[n - j]) : cmk<double>(0, 0);
-        dft_fold<true>(E, O, j, c, pr, x, m);
+    const int W = blockDim.x >> 6, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    for (int c = wave; c < DFT_LINES; c += W) {
+        const int yl = y0 + (c & 3);
+        const bool ok = (c < 4 ? hasA : hasB) && yl < a.ny;
+        dft_load_line<true>(P, n, 0, c, ok ? (c < 4 ? FA : FB) + (size_t)yl * n : nullptr, [](int, zd v) { return v; });
     }
-    const int W = blockDim.x >> 6, lane = threadIdx.x & 63;
+    if (idle) return;  // (the lines were loaded meanwhile)
+    if (a.count && blockIdx.x == 0 && threadIdx.x == 0) a.count[f] += 1;
     const int y = y0 + (lane >> 4);
     const bool oky = y < a.ny;
     const double yy = a.Y[oky ? y : 0];
     const bool fwd = (a.flags & DF_FWD) != 0;
     const int lo = fwd ? a.dft.lo : 0;  // the next aperture keeps the folded indices >= lo
     const int b0 = (b == a.R || (a.flags & DF_AMAX)) ? 0 : lo, a2 = lo & ~3;
-    int tile0, mt = dft_tiles(n, b0);
-    dbl4 e[TPW], o[TPW];
-    bool own = dft_stage<TPW>(E, O, part, n, 0, b0, mt, a.dft.smax, a.dft.tab, ld, e, o, tile0);
-    // boundary update (src/boost_fractor_recurprop.jl:90-119)
+    int mt = dft_tiles(n, b0);
+    DftShare sh(mt, a.dft.smax);
+    // what the update needs, loaded ahead of the transform
     const zd r = a.coef[b];
-    const zd omr = cmk<double>(1.0 - r.re, -r.im), opr = cmk<double>(1.0 + r.re, r.im), mr = cmk<double>(-r.re, -r.im);
     const int tA = a.rtab && hasA ? a.rtab_idx[f * a.R + b - 1] : -1, tB = a.rtab && hasB ? a.rtab_idx[f * a.R + b] : -1;
+    double xs[TPW][2];
+#pragma unroll
+    for (int q = 0; q < TPW; q++) {
+        const int j = b0 + 16 * (sh.first + q * W) + (lane & 15);
+        xs[q][0] = a.X[j <= H ? j : H];
+        xs[q][1] = a.X[j > 0 && j <= H ? n - j : 0];
+    }
+    dbl4 e[TPW], o[TPW];
+    dft_stage<TPW>(P, part, n, 0, b0, mt, sh, a.dft.tab, e, o);
+    // boundary update (src/boost_fractor_recurprop.jl:90-119)
+    const zd omr = cmk<double>(1.0 - r.re, -r.im), opr = cmk<double>(1.0 + r.re, r.im), mr = cmk<double>(-r.re, -r.im);
     double vmax = 0.0;
-    auto update = [&](int x, zd& A, zd& B) {
+    auto update = [&](int x, double xx, zd& A, zd& B) {
         const size_t p = (size_t)y * n + x;
         if (tA >= 0) A = cmul(A, ccast<double>(a.rtab[(size_t)tA * K + p]));
         if (tB >= 0) B = cmul(B, ccast<double>(a.rtab[(size_t)tB * K + p]));
@@ -280,21 +362,24 @@ __global__ void __launch_bounds__(1024) k_dancer_rows_dft(DancerRowArgs<T> a) {
         A = hasA ? nA : cmk<double>(0, 0);
         B = hasB ? nB : cmk<double>(0, 0);
         if (a.flags & DF_AMAX) vmax = fmax(vmax, fmax(hypot(A.re, A.im), hypot(B.re, B.im)));
-        if (fwd && !in_aperture(a.X[x], yy, a.R2)) A = B = cmk<double>(0, 0);  // next bounce's aperture
+        if (fwd && !in_aperture(xx, yy, a.R2)) A = B = cmk<double>(0, 0);  // next bounce's aperture
     };
-    if (own && oky)
+    if (sh.own(mt) && oky)
 #pragma unroll
         for (int q = 0; q < TPW; q++) {
-            const int j = b0 + 16 * (tile0 + q * W) + (lane & 15);
-            if (tile0 + q * W >= mt || j > H) continue;
+            const int j = b0 + 16 * (sh.first + q * W) + (lane & 15);
+            if (sh.first + q * W >= mt || j > H) continue;
             const bool pr = dft_paired(n, j);
             zd A = dft_out(e[q], o[q], 0), B = dft_out(e[q], o[q], 1);
             zd mA = dft_mirror(e[q], o[q], 0), mB = dft_mirror(e[q], o[q], 1);
-            update(j, A, B);
-            if (pr) update(n - j, mA, mB);
+            update(j, xs[q][0], A, B);
+            if (pr)
+                update(n - j, xs[q][1], mA, mB);
+            else
+                mA = mB = cmk<double>(0, 0);
             if (j >= lo) {
-                dft_fold<false>(E, O, j - a2, lane >> 4, pr, A, mA);
-                dft_fold<false>(E, O, j - a2, 4 + (lane >> 4), pr, B, mB);
+                dft_fold<false>(P, j - a2, lane >> 4, A, mA);
+                dft_fold<false>(P, j - a2, 4 + (lane >> 4), B, mB);
             }
         }
     if (a.flags & DF_AMAX) {
@@ -308,15 +393,16 @@ __global__ void __launch_bounds__(1024) k_dancer_rows_dft(DancerRowArgs<T> a) {
         }
     }
     if (!fwd || exit_only) return;  // only Eout is needed
-    dft_zero_rows(E, O, 0, lo - a2);
-    dft_zero_rows(E, O, H + 1 - a2, dft_rows(n, a2));
+    dft_zero_rows(P, 0, lo - a2);
+    dft_zero_rows(P, H + 1 - a2, dft_rows(n, a2));
     mt = dft_tiles(n, 0);
-    own = dft_stage<TPW>(E, O, part, n, a2, 0, mt, a.dft.smax, a.dft.tab, ld, e, o, tile0);
-    if (!own || !oky) return;
+    sh = DftShare(mt, a.dft.smax);
+    dft_stage<TPW>(P, part, n, a2, 0, mt, sh, a.dft.tab, e, o);
+    if (!sh.own(mt) || !oky) return;
 #pragma unroll
     for (int q = 0; q < TPW; q++) {
-        const int j = 16 * (tile0 + q * W) + (lane & 15);
-        if (tile0 + q * W >= mt || j > H) continue;
+        const int j = 16 * (sh.first + q * W) + (lane & 15);
+        if (sh.first + q * W >= mt || j > H) continue;
 #pragma unroll
         for (int h = 0; h < 2; h++) {
             if (!(h == 0 ? hasA : hasB)) continue;
@@ -328,14 +414,18 @@ __global__ void __launch_bounds__(1024) k_dancer_rows_dft(DancerRowArgs<T> a) {
 }
 
 // The pair step on the matrix cores: 4 rows, lines 0..3 field i, 4..7 field i+1
+template <typename T>
+struct ChPairDftArgs : ChPairArgs<T> {
+    int n;
+};
+
 template <typename T, int TPW>
-__global__ void __launch_bounds__(1024) k_ch_pair_dft(ChPairArgs<T> a, int n) {
+__global__ void __launch_bounds__(1024) k_ch_pair_dft(ChPairDftArgs<T> a) {
     using S = typename Storage<T>::type;
-    extern __shared__ unsigned char smem_raw[];
-    const int H = n >> 1, ld = dft_ld(n);
-    double* E = reinterpret_cast<double*>(smem_raw);
-    double* O = E + dft_rows(n, 0) * DFT_LDP;
-    double* part = O + dft_rows(n, 0) * DFT_LDP;
+    extern __shared__ double2 dft_smem[];
+    const int n = a.n, H = n >> 1;
+    double2* P = dft_smem;
+    double2* part = P + dft_rows(n, 0) * DFT_LDP;
     const int en = blockIdx.y;
     const FieldDesc d0 = a.fd[2 * en], d1 = a.fd[2 * en + 1];
     if (a.active && !a.active[d0.group]) return;  // uniform over the block
@@ -343,29 +433,34 @@ __global__ void __launch_bounds__(1024) k_ch_pair_dft(ChPairArgs<T> a, int n) {
     const int y0 = a.ylo + blockIdx.x * 4;
     cplx<S>* F0 = a.F + d0.off;
     cplx<S>* F1 = a.F + d1.off;
-    const int rows = dft_rows(n, 0);
-    for (int q = threadIdx.x; q < rows * DFT_LINES; q += blockDim.x) {
-        const int c = q / rows, j = q - c * rows, y = y0 + (c & 3);
-        const bool ok = y < a.yhi && j <= H, pr = dft_paired(n, j);
-        const cplx<S>* row = (c < 4 ? F0 : F1) + (size_t)y * n;
-        const zd x = ok ? ccast<double>(row[j]) : cmk<double>(0, 0);
-        const zd m = ok && pr ? ccast<double>(row[n - j]) : cmk<double>(0, 0);
-        dft_fold<true>(E, O, j, c, pr, x, m);
+    const int W = blockDim.x >> 6, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    for (int c = wave; c < DFT_LINES; c += W) {
+        const int yl = y0 + (c & 3);
+        dft_load_line<true>(P, n, 0, c, yl < a.yhi ? (c < 4 ? F0 : F1) + (size_t)yl * n : nullptr,
+                            [](int, zd v) { return v; });
     }
-    const int W = blockDim.x >> 6, lane = threadIdx.x & 63;
     const int y = y0 + (lane >> 4);
     const bool oky = y < a.yhi;
     const double yy = a.Y[oky ? y : 0];
     const bool xout = a.xout != 0;
     const int lo = xout ? a.dft.lo : 0, a2 = lo & ~3;  // the mask of the next transform keeps the folded indices >= lo
-    int tile0, mt = dft_tiles(n, lo);
-    dbl4 e[TPW], o[TPW];
-    bool own = dft_stage<TPW>(E, O, part, n, 0, lo, mt, a.dft.smax, a.dft.tab, ld, e, o, tile0);
+    int mt = dft_tiles(n, lo);
+    DftShare sh(mt, a.dft.smax);
+    // what the update needs, loaded ahead of the transform
     const zd* cf = a.coef + 4 * (d0.pad >> FD_PAIR_SHIFT);
     const zd rl = cf[0], tr = cf[1], rr = cf[2], tl = cf[3];
+    double xs[TPW][2];
+#pragma unroll
+    for (int q = 0; q < TPW; q++) {
+        const int j = lo + 16 * (sh.first + q * W) + (lane & 15);
+        xs[q][0] = a.X[j <= H ? j : H];
+        xs[q][1] = a.X[j > 0 && j <= H ? n - j : 0];
+    }
+    dbl4 e[TPW], o[TPW];
+    dft_stage<TPW>(P, part, n, 0, lo, mt, sh, a.dft.tab, e, o);
     const int t0 = a.rtab ? d0.rtab : -1, t1 = a.rtab ? d1.rtab : -1;
     // k_ch_pair: Fn = c rl + tr a, Fi = a rr + tl c (a: field i, c: field i+1), rounded as they are stored
-    auto update = [&](int x, zd& A, zd& B) {
+    auto update = [&](int x, double xx, zd& A, zd& B) {
         const size_t p = (size_t)y * n + x;
         if (t0 >= 0) A = cmul(A, ccast<double>(a.rtab[(size_t)t0 * K + p]));
         if (t1 >= 0) B = cmul(B, ccast<double>(a.rtab[(size_t)t1 * K + p]));
@@ -374,21 +469,24 @@ __global__ void __launch_bounds__(1024) k_ch_pair_dft(ChPairArgs<T> a, int n) {
         const zd nA = cadd(cmul(A, rr), cmul(tl, B)), nB = cadd(cmul(B, rl), cmul(tr, A));
         A = ccast<double>(ccast<S>(nA));
         B = ccast<double>(ccast<S>(nB));
-        if (xout && !in_aperture(a.X[x], yy, a.R2)) A = B = cmk<double>(0, 0);
+        if (xout && !in_aperture(xx, yy, a.R2)) A = B = cmk<double>(0, 0);
     };
-    if (own && oky)
+    if (sh.own(mt) && oky)
 #pragma unroll
         for (int q = 0; q < TPW; q++) {
-            const int j = lo + 16 * (tile0 + q * W) + (lane & 15);
-            if (tile0 + q * W >= mt || j > H) continue;
+            const int j = lo + 16 * (sh.first + q * W) + (lane & 15);
+            if (sh.first + q * W >= mt || j > H) continue;
             const bool pr = dft_paired(n, j);
             zd A = dft_out(e[q], o[q], 0), B = dft_out(e[q], o[q], 1);
             zd mA = dft_mirror(e[q], o[q], 0), mB = dft_mirror(e[q], o[q], 1);
-            update(j, A, B);
-            if (pr) update(n - j, mA, mB);
+            update(j, xs[q][0], A, B);
+            if (pr)
+                update(n - j, xs[q][1], mA, mB);
+            else
+                mA = mB = cmk<double>(0, 0);
             if (xout) {
-                dft_fold<false>(E, O, j - a2, lane >> 4, pr, A, mA);
-                dft_fold<false>(E, O, j - a2, 4 + (lane >> 4), pr, B, mB);
+                dft_fold<false>(P, j - a2, lane >> 4, A, mA);
+                dft_fold<false>(P, j - a2, 4 + (lane >> 4), B, mB);
             } else {
                 cplx<S>* r0 = F0 + (size_t)y * n;
                 cplx<S>* r1 = F1 + (size_t)y * n;
@@ -401,15 +499,16 @@ __global__ void __launch_bounds__(1024) k_ch_pair_dft(ChPairArgs<T> a, int n) {
             }
         }
     if (!xout) return;
-    dft_zero_rows(E, O, 0, lo - a2);
-    dft_zero_rows(E, O, H + 1 - a2, dft_rows(n, a2));
+    dft_zero_rows(P, 0, lo - a2);
+    dft_zero_rows(P, H + 1 - a2, dft_rows(n, a2));
     mt = dft_tiles(n, 0);
-    own = dft_stage<TPW>(E, O, part, n, a2, 0, mt, a.dft.smax, a.dft.tab, ld, e, o, tile0);
-    if (!own || !oky) return;
+    sh = DftShare(mt, a.dft.smax);
+    dft_stage<TPW>(P, part, n, a2, 0, mt, sh, a.dft.tab, e, o);
+    if (!sh.own(mt) || !oky) return;
 #pragma unroll
     for (int q = 0; q < TPW; q++) {
-        const int j = 16 * (tile0 + q * W) + (lane & 15);
-        if (tile0 + q * W >= mt || j > H) continue;
+        const int j = 16 * (sh.first + q * W) + (lane & 15);
+        if (sh.first + q * W >= mt || j > H) continue;
 #pragma unroll
         for (int h = 0; h < 2; h++) {
             cplx<S>* row = (h == 0 ? F0 : F1) + (size_t)y * n;
@@ -431,23 +530,18 @@ struct DftShape {
         tpw = mt <= 16 ? 1 : 2;
         waves = (mt + tpw - 1) / tpw;
         if (waves > 2) waves = (waves + 3) & ~3;  // whole rounds over the four SIMDs
-        const size_t planes = sizeof(double) * 2 * DFT_LDP * (size_t)dft_rows(n, 0);
-        const size_t part = sizeof(double) * DFT_PART * (size_t)(waves - 1);
+        const size_t planes = sizeof(double2) * DFT_LDP * (size_t)dft_rows(n, 0);
+        const size_t part = sizeof(double2) * DFT_PART * (size_t)(waves - 1);
         const bool share = planes + part <= 152 * 1024;
         smax = share ? 4 : 1;
         smem = planes + (share ? part : 0);
     }
 };
-#define BF_DFT_LAUNCH(kernel, T, sh, grid, s, ...)                                                                  \
-    do {                                                                                                             \
-        if ((sh).tpw == 1) {                                                                                         \
-            allow_lds((const void*)kernel<T, 1>, (sh).smem);                                                         \
-            hipLaunchKernelGGL((kernel<T, 1>), grid, dim3(64 * (sh).waves), (sh).smem, s, __VA_ARGS__);              \
-        } else {                                                                                                     \
-            allow_lds((const void*)kernel<T, 2>, (sh).smem);                                                         \
-            hipLaunchKernelGGL((kernel<T, 2>), grid, dim3(64 * (sh).waves), (sh).smem, s, __VA_ARGS__);              \
-        }                                                                                                            \
-        BF_CHECK_LAUNCH();                                                                                           \
+#define BF_DFT_GO(grid, sh, s, arg, ...)                                                          \
+    do {                                                                                          \
+        allow_lds((const void*)__VA_ARGS__, (sh).smem);                                           \
+        hipLaunchKernelGGL((__VA_ARGS__), grid, dim3(64 * (sh).waves), (sh).smem, s, arg);        \
+        BF_CHECK_LAUNCH();                                                                        \
     } while (0)
 
 template <typename T>
@@ -455,27 +549,54 @@ void launch_rows_dft(RowArgs<T> a, hipStream_t s) {
     const DftShape sh(a.nx);
     a.dft.smax = sh.smax;
     const long nlines = (long)a.nf * (a.yhi > a.ylo ? a.yhi - a.ylo : a.ny);
-    BF_DFT_LAUNCH(k_rows_dft, T, sh, dim3((unsigned)((nlines + DFT_LINES - 1) / DFT_LINES)), s, a);
+    if (nlines > 0x7fffffffL - DFT_LINES) throw Error(BF_ERR_UNSUPPORTED, "too many lines in one row pass");
+    const dim3 grid((unsigned)((nlines + DFT_LINES - 1) / DFT_LINES));
+    if (sh.tpw == 1)
+        BF_DFT_GO(grid, sh, s, a, k_rows_dft<T, 1>);
+    else
+        BF_DFT_GO(grid, sh, s, a, k_rows_dft<T, 2>);
 }
 template <typename T>
 void launch_cols_dft(ColArgs<T> a, hipStream_t s) {
     const DftShape sh(a.ny);
     a.dft.smax = sh.smax;
-    BF_DFT_LAUNCH(k_cols_dft, T, sh, dim3((a.nx + DFT_LINES - 1) / DFT_LINES, a.nf), s, a);
+    constexpr uint32_t PROP = CF_FWD | CF_KMID | CF_INV;
+    const dim3 grid((a.nx + DFT_LINES - 1) / DFT_LINES, a.nf);
+    if (a.flags == PROP && a.ktab) {
+        if (sh.tpw == 1)
+            BF_DFT_GO(grid, sh, s, a, k_cols_dft<T, 1, PROP>);
+        else
+            BF_DFT_GO(grid, sh, s, a, k_cols_dft<T, 2, PROP>);
+    } else {
+        if (sh.tpw == 1)
+            BF_DFT_GO(grid, sh, s, a, k_cols_dft<T, 1, 0>);
+        else
+            BF_DFT_GO(grid, sh, s, a, k_cols_dft<T, 2, 0>);
+    }
 }
 template <typename T>
 void launch_dancer_rows_dft(DancerRowArgs<T> a, int fb, hipStream_t s) {
     const DftShape sh(a.nx);
     a.dft.smax = sh.smax;
     const unsigned nblk = dancer_tiles(a, 4);
-    BF_DFT_LAUNCH(k_dancer_rows_dft, T, sh, dim3(nblk, fb), s, a);
+    if (sh.tpw == 1)
+        BF_DFT_GO(dim3(nblk, fb), sh, s, a, k_dancer_rows_dft<T, 1>);
+    else
+        BF_DFT_GO(dim3(nblk, fb), sh, s, a, k_dancer_rows_dft<T, 2>);
 }
 template <typename T>
 void launch_ch_pair_dft(ChPairArgs<T> a, int nx, int entries, hipStream_t s) {
     if (!a.dft.tab) throw std::runtime_error("the pair step's row transforms have no table");
     const DftShape sh(nx);
     a.dft.smax = sh.smax;
-    BF_DFT_LAUNCH(k_ch_pair_dft, T, sh, dim3((a.yhi - a.ylo + 3) / 4, entries), s, a, nx);
+    ChPairDftArgs<T> b;
+    static_cast<ChPairArgs<T>&>(b) = a;
+    b.n = nx;
+    const dim3 grid((a.yhi - a.ylo + 3) / 4, entries);
+    if (sh.tpw == 1)
+        BF_DFT_GO(grid, sh, s, b, k_ch_pair_dft<T, 1>);
+    else
+        BF_DFT_GO(grid, sh, s, b, k_ch_pair_dft<T, 2>);
 }
 #define BF_DFT_INSTANCES(T)                                                     \
     template void launch_rows_dft<T>(RowArgs<T>, hipStream_t);                  \
@@ -485,16 +606,16 @@ void launch_ch_pair_dft(ChPairArgs<T> a, int nx, int entries, hipStream_t s) {
 BF_DFT_INSTANCES(double)
 BF_DFT_INSTANCES(float)
 
-// (cos, sin)(2 pi a b / n) for the matrix-core line transforms, a, b < dft_ld(n)
-__global__ void k_dft_table(double2* out, int n, int ld) {
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < ld * ld; i += gridDim.x * blockDim.x) {
+// (cos, sin)(2 pi a b / n) for the matrix-core line transforms, a < dft_tab_rows(n), b < dft_ld(n)
+__global__ void k_dft_table(double2* out, int n, int ld, int rows) {
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < ld * rows; i += gridDim.x * blockDim.x) {
         const int m = (int)(((long)(i / ld) * (i % ld)) % n);
         double s, c;
         sincospi(2.0 * (double)m / (double)n, &s, &c);
         out[i] = make_double2(c, s);
     }
 }
-// The context keeps the tables of the last lengths used (at most 4.4 MB each, n = 1023); an
+// The context keeps the tables of the last lengths used (at most 4.7 MB each, n = 1023); an
 // engine holds its own reference, so a table dropped here lives as long as a plan that reads it.
 std::shared_ptr<DevBuf> dft_table(bf_ctx* ctx, int n) {
     auto& cache = ctx->dft_tables;
@@ -503,9 +624,10 @@ std::shared_ptr<DevBuf> dft_table(bf_ctx* ctx, int n) {
             std::rotate(cache.begin() + q, cache.begin() + q + 1, cache.end());
             return cache.back().second;
         }
-    const int ld = dft_ld(n);
-    auto b = std::make_shared<DevBuf>(sizeof(double2) * (size_t)ld * ld);
-    hipLaunchKernelGGL(k_dft_table, dim3((ld * ld + 255) / 256), dim3(256), 0, ctx->stream, b->as<double2>(), n, ld);
+    const int ld = dft_ld(n), rows = dft_tab_rows(n);
+    auto b = std::make_shared<DevBuf>(sizeof(double2) * (size_t)ld * rows);
+    hipLaunchKernelGGL(k_dft_table, dim3((ld * rows + 255) / 256), dim3(256), 0, ctx->stream, b->as<double2>(), n, ld,
+                       rows);
     BF_CHECK_LAUNCH();
     if (cache.size() >= 8) cache.erase(cache.begin());
     cache.emplace_back(n, b);
