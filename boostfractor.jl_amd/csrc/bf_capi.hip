@@ -28,13 +28,24 @@ static int fail(const bf_ctx* ctx, int code, const std::string& msg) {
     } while (0)
 
 namespace bf {
-static thread_local const EngineOptions* t_opt = nullptr;
+static thread_local bf_ctx* t_call = nullptr;
 const EngineOptions& opts() {
     static const EngineOptions defaults;
-    return t_opt ? *t_opt : defaults;
+    return t_call ? t_call->opt : defaults;
 }
-OptionScope::OptionScope(const EngineOptions* o) : prev(t_opt) { t_opt = o; }
-OptionScope::~OptionScope() { t_opt = prev; }
+const std::shared_ptr<DevPool>& call_pool() {
+    static const std::shared_ptr<DevPool> none;
+    return t_call ? t_call->pool : none;
+}
+CallScope::CallScope(bf_ctx* c) : prev(t_call) { t_call = c; }
+CallScope::~CallScope() { t_call = prev; }
+void upload(void* dst, const void* src, size_t bytes, hipStream_t s) {
+    if (!bytes) return;
+    if (t_call && s == t_call->stream && bytes <= UploadRing::MOST)
+        t_call->ring.put(dst, src, bytes, s);
+    else
+        BF_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, s));
+}
 }  // namespace bf
 
 namespace bf {
@@ -53,7 +64,7 @@ void save_tuned(bf_ctx* ctx, const std::string& key) {
 template <typename F>
 static int guarded(bf_ctx* ctx, F&& body) {
     try {
-        bf::OptionScope scope(ctx ? &ctx->opt : nullptr);
+        bf::CallScope scope(ctx);
         if (ctx) BF_HIP(hipSetDevice(ctx->device));
         body();
         return BF_OK;
@@ -164,6 +175,8 @@ int bf_ctx_destroy(bf_ctx* ctx) {
     bf::clear_timers(ctx);
     ctx->twiddles.clear();
     ctx->dft_tables.clear();
+    ctx->scratch.clear();
+    ctx->pool->trim(true);  // blocks of plans that outlive the context are freed by them
     if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
     delete ctx;
     return BF_OK;

@@ -855,9 +855,6 @@ void allow_lds(const void* kernel, size_t bytes) {
     BF_HIP(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes));
 }
 
-void upload(void* dst, const void* src, size_t bytes, hipStream_t s) {
-    if (bytes) BF_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, s));
-}
 void download(void* dst, const void* src, size_t bytes, hipStream_t s) {
     if (bytes) BF_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s));
 }
@@ -865,14 +862,19 @@ void download(void* dst, const void* src, size_t bytes, hipStream_t s) {
 void Grid::upload(const bf_coords* c, hipStream_t s) {
     nx = c->nx;
     ny = c->ny;
-    X.alloc(sizeof(double) * nx);
-    Y.alloc(sizeof(double) * ny);
-    kX.alloc(sizeof(double) * nx);
-    kY.alloc(sizeof(double) * ny);
-    bf::upload(X.p, c->X, sizeof(double) * nx, s);
-    bf::upload(Y.p, c->Y, sizeof(double) * ny, s);
-    bf::upload(kX.p, c->kX, sizeof(double) * nx, s);
-    bf::upload(kY.p, c->kY, sizeof(double) * ny, s);
+    const int len[4] = {nx, ny, nx, ny};
+    const double* src[4] = {c->X, c->Y, c->kX, c->kY};
+    View* view[4] = {&X, &Y, &kX, &kY};
+    std::vector<double> all;
+    all.reserve(2 * (size_t)(nx + ny));
+    for (int q = 0; q < 4; q++) all.insert(all.end(), src[q], src[q] + len[q]);
+    axes.alloc(sizeof(double) * all.size());
+    bf::upload(axes.p, all.data(), sizeof(double) * all.size(), s);
+    double* d = axes.as<double>();
+    for (int q = 0; q < 4; q++) {
+        view[q]->p = d;
+        d += len[q];
+    }
     hX.assign(c->X, c->X + nx);
     hY.assign(c->Y, c->Y + ny);
     hkX.assign(c->kX, c->kX + nx);

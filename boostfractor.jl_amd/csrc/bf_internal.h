@@ -6,7 +6,9 @@
 #include <cstdint>
 #include <cstring>
 #include <map>
+#include <iterator>
 #include <memory>
+#include <mutex>
 #include <stdexcept>
 #include <string>
 #include <utility>
@@ -33,6 +35,72 @@ struct Error : std::runtime_error {
 
 #define BF_CHECK_LAUNCH() BF_HIP(hipGetLastError())
 
+// Device memory given back by the buffers of one context, for its next ones.  A call
+// allocates a dozen buffers and frees them when it returns; hipMalloc and hipFree take
+// ~9 us each (milliseconds for hundreds of MB, and hipFree waits for the device).
+// Everything a context does is ordered on its one stream, so memory that work queued
+// earlier may still use can be handed out again at once.  The pool keeps at most
+// KEEP bytes (the smallest blocks first), frees them all when an allocation fails and
+// when the context is destroyed; blocks that come back later are freed directly.
+// A plan may be destroyed on another thread than its context's calls: the lock.
+class DevPool {
+  public:
+    static constexpr size_t KEEP = (size_t)2 << 30;
+    // block sizes: multiples of an eighth of the next lower power of two (at least 512 bytes)
+    static size_t round(size_t n) {
+        size_t g = 512;
+        while (g * 16 <= n) g *= 2;
+        return (n + g - 1) / g * g;
+    }
+    void* take(size_t block) {
+        std::lock_guard<std::mutex> lk(mu);
+        auto it = blocks.find(block);
+        if (it == blocks.end()) return nullptr;
+        void* p = it->second;
+        blocks.erase(it);
+        kept -= block;
+        return p;
+    }
+    void give(void* p, size_t block) {
+        std::vector<void*> out;
+        {
+            std::lock_guard<std::mutex> lk(mu);
+            if (closed || block > KEEP) {
+                out.push_back(p);
+            } else {
+                blocks.emplace(block, p);
+                kept += block;
+                while (kept > KEEP) {  // the largest go
+                    auto it = std::prev(blocks.end());
+                    out.push_back(it->second);
+                    kept -= it->first;
+                    blocks.erase(it);
+                }
+            }
+        }
+        for (void* q : out) (void)hipFree(q);
+    }
+    void trim(bool close = false) {
+        std::multimap<size_t, void*> out;
+        {
+            std::lock_guard<std::mutex> lk(mu);
+            out.swap(blocks);
+            kept = 0;
+            closed = closed || close;
+        }
+        for (auto& b : out) (void)hipFree(b.second);
+    }
+    ~DevPool() { trim(true); }
+
+  private:
+    std::mutex mu;
+    std::multimap<size_t, void*> blocks;
+    size_t kept = 0;
+    bool closed = false;
+};
+// pool of the context whose call runs on this thread (null outside a call)
+const std::shared_ptr<DevPool>& call_pool();
+
 // Owning device allocation.
 struct DevBuf {
     void* p = nullptr;
@@ -41,30 +109,63 @@ struct DevBuf {
     explicit DevBuf(size_t n) { alloc(n); }
     DevBuf(const DevBuf&) = delete;
     DevBuf& operator=(const DevBuf&) = delete;
-    DevBuf(DevBuf&& o) noexcept : p(o.p), bytes(o.bytes) { o.p = nullptr; o.bytes = 0; }
+    DevBuf(DevBuf&& o) noexcept : p(o.p), bytes(o.bytes), block(o.block), pool(std::move(o.pool)) {
+        o.p = nullptr;
+        o.bytes = 0;
+    }
     DevBuf& operator=(DevBuf&& o) noexcept {
-        if (this != &o) { release(); p = o.p; bytes = o.bytes; o.p = nullptr; o.bytes = 0; }
+        if (this != &o) {
+            release();
+            p = o.p;
+            bytes = o.bytes;
+            block = o.block;
+            pool = std::move(o.pool);
+            o.p = nullptr;
+            o.bytes = 0;
+        }
         return *this;
     }
     ~DevBuf() { release(); }
     void alloc(size_t n) {
         release();
         if (n == 0) return;
-        hipError_t e = hipMalloc(&p, n);
-        if (e != hipSuccess) {
-            p = nullptr;
-            throw Error(e == hipErrorOutOfMemory ? BF_ERR_NOMEM : BF_ERR_HIP,
-                        std::string("hipMalloc(") + std::to_string(n) + " bytes): " + hipGetErrorString(e));
+        pool = call_pool();
+        block = pool ? DevPool::round(n) : n;
+        if (pool) p = pool->take(block);
+        if (!p) {
+            hipError_t e = hipMalloc(&p, block);
+            if (e == hipErrorOutOfMemory && pool) {  // what the pool keeps, and the rounding, may be what is missing
+                (void)hipGetLastError();
+                pool->trim();
+                block = n;
+                e = hipMalloc(&p, block);
+            }
+            if (e != hipSuccess) {
+                p = nullptr;
+                pool.reset();
+                throw Error(e == hipErrorOutOfMemory ? BF_ERR_NOMEM : BF_ERR_HIP,
+                            std::string("hipMalloc(") + std::to_string(n) + " bytes): " + hipGetErrorString(e));
+            }
         }
         bytes = n;
     }
     void release() {
-        if (p) (void)hipFree(p);
+        if (p) {
+            if (pool)
+                pool->give(p, block);
+            else
+                (void)hipFree(p);
+        }
         p = nullptr;
         bytes = 0;
+        pool.reset();
     }
     template <typename U>
     U* as() const { return static_cast<U*>(p); }
+
+  private:
+    size_t block = 0;  // bytes allocated
+    std::shared_ptr<DevPool> pool;
 };
 
 }  // namespace bf
@@ -113,19 +214,67 @@ struct EngineOptions {
 };
 // Options of the context whose call runs on this thread (defaults outside a call).
 const EngineOptions& opts();
-// Makes `o` the running call's options for the lifetime of the object.
-struct OptionScope {
-    const EngineOptions* prev;
-    explicit OptionScope(const EngineOptions* o);
-    ~OptionScope();
-    OptionScope(const OptionScope&) = delete;
-    OptionScope& operator=(const OptionScope&) = delete;
+// Makes `c` the context of the running call (its options, device memory and staging
+// memory) for the lifetime of the object.
+struct CallScope {
+    bf_ctx* prev;
+    explicit CallScope(bf_ctx* c);
+    ~CallScope();
+    CallScope(const CallScope&) = delete;
+    CallScope& operator=(const CallScope&) = delete;
+};
+
+// Pinned memory that small uploads are copied through: the caller's bytes are taken
+// when put() returns, as with pageable memory, without the runtime's wait for them
+// (18 against ~3 us a call).  Two halves; a half is reused once the copies queued from
+// it are done.  One per context, used by the context's calls only.
+class UploadRing {
+  public:
+    static constexpr size_t HALF = (size_t)1 << 20, MOST = (size_t)64 << 10;
+    UploadRing() = default;
+    UploadRing(const UploadRing&) = delete;
+    UploadRing& operator=(const UploadRing&) = delete;
+    ~UploadRing() {
+        for (int h = 0; h < 2; h++)
+            if (done[h]) {
+                (void)hipEventSynchronize(done[h]);
+                (void)hipEventDestroy(done[h]);
+            }
+        if (base) (void)hipHostFree(base);
+    }
+    void put(void* dst, const void* src, size_t bytes, hipStream_t s) {
+        if (!base) {
+            void* p = nullptr;
+            BF_HIP(hipHostMalloc(&p, 2 * HALF));
+            base = static_cast<char*>(p);
+        }
+        const size_t need = (bytes + 63) & ~(size_t)63;
+        if (used + need > HALF) {
+            if (!done[cur]) BF_HIP(hipEventCreateWithFlags(&done[cur], hipEventDisableTiming));
+            BF_HIP(hipEventRecord(done[cur], s));
+            cur ^= 1;
+            used = 0;
+            if (done[cur]) BF_HIP(hipEventSynchronize(done[cur]));
+        }
+        char* h = base + cur * HALF + used;
+        std::memcpy(h, src, bytes);
+        BF_HIP(hipMemcpyAsync(dst, h, bytes, hipMemcpyHostToDevice, s));
+        used += need;
+    }
+
+  private:
+    char* base = nullptr;
+    size_t used = 0;
+    int cur = 0;
+    hipEvent_t done[2] = {nullptr, nullptr};
 };
 }  // namespace bf
 
 // Per-caller context: one device, one stream, cached twiddle tables.
 struct bf_ctx {
     bf::EngineOptions opt;
+    std::shared_ptr<bf::DevPool> pool = std::make_shared<bf::DevPool>();
+    bf::UploadRing ring;
     int device = 0;
     hipStream_t stream = nullptr;
     std::string err;
@@ -272,8 +421,14 @@ void clear_timers(bf_ctx* ctx);
 
 // Device-resident coordinate grids.
 struct Grid {
+    struct View {
+        double* p = nullptr;
+        template <typename U>
+        U* as() const { return p; }
+    };
     int nx = 0, ny = 0;
-    DevBuf X, Y, kX, kY;  // double
+    DevBuf axes;         // X, Y, kX, kY, double: one upload
+    View X, Y, kX, kY;
     std::vector<double> hX, hY, hkX, hkY;  // host copies
     void upload(const bf_coords* c, hipStream_t s);
     size_t K() const { return (size_t)nx * ny; }
