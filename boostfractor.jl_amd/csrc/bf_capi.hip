@@ -214,6 +214,7 @@ static int64_t* option_slot(bf::EngineOptions& o, const char* name, int64_t& tmp
     static const Int ints[] = {
         {"fft_lds", &bf::EngineOptions::fft_lds}, {"prune", &bf::EngineOptions::prune},
         {"qtab", &bf::EngineOptions::qtab}, {"band", &bf::EngineOptions::band},
+        {"reduced", &bf::EngineOptions::reduced},
         {"chfuse", &bf::EngineOptions::chfuse}, {"chxf", &bf::EngineOptions::chxf},
         {"chwave", &bf::EngineOptions::chwave}, {"graph", &bf::EngineOptions::graph},
         {"col_tx", &bf::EngineOptions::col_tx}, {"rows", &bf::EngineOptions::rows},

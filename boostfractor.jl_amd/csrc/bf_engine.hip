@@ -17,6 +17,7 @@
 // reading and writing every field once.  The per-region k-space phase tables
 // are built once per frequency batch from FP64 arguments.
 #include "bf_passes.h"
+#include "bf_reduced.h"
 #include "bf_fftreg.h"
 
 #include <algorithm>
@@ -1298,6 +1299,123 @@ static zd phase_1d(zd eps, double lambda, double dz) {
 }
 
 // ---------------------------------------------------------------------------
+// propagation on the aperture's window (bf_reduced.h)
+// ---------------------------------------------------------------------------
+// What a bounce solver on the window needs besides its fields: the window, the tables
+// of the reduced convolution and the whole-grid propagation of the sums.
+struct Reduced {
+    // bounces below which the tables cost more than the smaller transforms save: a table
+    // takes two transforms of the grid, a bounce two smaller ones per field of ~4 per table
+    static constexpr int MIN_BOUNCES = 8;
+    bf_ctx* ctx;
+    const Grid* g;
+    RdShape sh;
+    Grid gm;  // the reduced grid: sizes only
+    std::unique_ptr<PropEngine<double>> pn, pm;  // whole grid; reduced grid
+    DevBuf tabs, keep, twx, twy, sum, fdn, fdm, fdout;
+
+    // The window of the grid's aperture, when the reduced convolution is at most 3/4 of the
+    // grid (a power of two) or no larger than it (other sizes, whose own lines take 2 n^2
+    // flop on the matrix cores): below that the smaller lines win at every size measured.
+    static bool shape(const Grid& g, double diskR, RdShape& sh) {
+        int lo, hi;
+        aperture_range(g.hY, g.hX, diskR, lo, hi);
+        sh.y0 = lo;
+        sh.by = hi - lo;
+        aperture_range(g.hX, g.hY, diskR, lo, hi);
+        sh.x0 = lo;
+        sh.bx = hi - lo;
+        if (sh.by <= 0 || sh.bx <= 0) return false;
+        sh.Ry = rd_radix(sh.by);
+        sh.Rx = rd_radix(sh.bx);
+        if (!sh.Ry || !sh.Rx) return false;
+        const bool pow2 = !dft_length(g.nx) && !dft_length(g.ny);
+        return pow2 ? 4 * sh.table() <= 3 * g.K() : sh.table() <= g.K();
+    }
+    static bool usable(const Grid& g, int kind, double amin, int nmax, double diskR, RdShape& sh) {
+        return opts().reduced && use_reg_fft() && amin == 0.0 && nmax + 1 >= MIN_BOUNCES &&
+               (kind == BF_PROP_PROPAGATOR || kind == BF_PROP_NOTILTS) && shape(g, diskR, sh);
+    }
+
+    Reduced(bf_ctx* c, const Grid* gr, const RdShape& s, int kind, double diskR, const zd* surfaces)
+        : ctx(c), g(gr), sh(s) {
+        gm.nx = sh.Mx();
+        gm.ny = sh.My();
+        pn.reset(new PropEngine<double>(ctx, g, kind, diskR, surfaces));
+        pn->blo = sh.y0;
+        pn->bhi = sh.y0 + sh.by;
+        pm.reset(new PropEngine<double>(ctx, &gm, BF_PROP_NOTILTS, diskR, nullptr));
+        std::vector<uint32_t> kb((size_t)sh.by * 16, 0u);
+        for (int y = 0; y < sh.by; y++)
+            for (int x = 0; x < sh.bx; x++)
+                if (in_aperture(g->hX[sh.x0 + x], g->hY[sh.y0 + y], diskR * diskR))
+                    kb[(size_t)y * 16 + x % 16] |= 1u << (x / 16);
+        keep.alloc(sizeof(uint32_t) * kb.size());
+        upload(keep.p, kb.data(), sizeof(uint32_t) * kb.size(), ctx->stream);
+        twx.alloc(sizeof(zd) * sh.Mx());
+        twy.alloc(sizeof(zd) * sh.My());
+        rd_twiddles(sh.Rx, twx.as<zd>(), ctx->stream);
+        rd_twiddles(sh.Ry, twy.as<zd>(), ctx->stream);
+    }
+
+    // T: ntab phase tables of the whole grid (times 1/K), overwritten -> tabs
+    void tables(zd* T, int ntab) {
+        const size_t K = g->K();
+        std::vector<FieldDesc> a(ntab), b(ntab);
+        for (int j = 0; j < ntab; j++) {
+            a[j] = FieldDesc{(int64_t)j * (int64_t)K, -1, -1, 0, 0};
+            b[j] = FieldDesc{(int64_t)j * (int64_t)sh.table(), -1, -1, 0, 0};
+        }
+        auto put = [&](DevBuf& d, const std::vector<FieldDesc>& v) {
+            if (d.bytes < sizeof(FieldDesc) * v.size()) d.alloc(sizeof(FieldDesc) * v.size());
+            upload(d.p, v.data(), sizeof(FieldDesc) * v.size(), ctx->stream);
+        };
+        put(fdn, a);
+        put(fdm, b);
+        if (tabs.bytes < sizeof(zd) * sh.table() * ntab) tabs.alloc(sizeof(zd) * sh.table() * ntab);
+        pn->rows(T, fdn.as<FieldDesc>(), ntab, RF_INV, nullptr);
+        pn->cols(T, T, fdn.as<FieldDesc>(), ntab, CF_INV, nullptr);
+        rd_crop(sh, T, g->nx, g->ny, ntab, tabs.as<zd>(), ctx->stream);
+        pm->rows(tabs.as<zd>(), fdm.as<FieldDesc>(), ntab, RF_FWD, nullptr);
+        pm->cols(tabs.as<zd>(), tabs.as<zd>(), fdm.as<FieldDesc>(), ntab, CF_FWD, nullptr);
+    }
+    void clear_sums(int n) {
+        const size_t bytes = sizeof(zd) * sh.field() * n;
+        if (sum.bytes < bytes) sum.alloc(bytes);
+        BF_HIP(hipMemsetAsync(sum.p, 0, bytes, ctx->stream));
+    }
+    // out[j] = propagation of sum slot0 + j by region regs[j] on the whole grid
+    void propagate_sums(int slot0, const std::vector<RegionParams>& regs, zd* out) {
+        const size_t K = g->K();
+        const int n = (int)regs.size();
+        BF_HIP(hipMemsetAsync(out, 0, sizeof(zd) * K * n, ctx->stream));
+        RdFinalArgs fa{sum.as<zd>() + (size_t)slot0 * sh.field(), out, sh.by, sh.bx, sh.x0, sh.y0, g->nx, K, twx.as<zd>()};
+        rd_final(sh, fa, n, ctx->stream);
+        pn->build_tables(regs);
+        std::vector<FieldDesc> fd(n);
+        for (int j = 0; j < n; j++)
+            fd[j] = FieldDesc{(int64_t)j * (int64_t)K, pn->ktab_of[j], pn->rtab_of.empty() ? -1 : pn->rtab_of[j], 0, 0};
+        if (fdout.bytes < sizeof(FieldDesc) * n) fdout.alloc(sizeof(FieldDesc) * n);
+        upload(fdout.p, fd.data(), sizeof(FieldDesc) * n, ctx->stream);
+        pn->propagate(out, fdout.as<FieldDesc>(), n, nullptr, nullptr, nullptr);
+    }
+    template <typename S>
+    RdColArgs<S> col_args(cplx<S>* F, const FieldDesc* fd) const {
+        return RdColArgs<S>{F, fd, sh.Mx(), sh.by, tabs.as<zd>(), sum.as<zd>(), twy.as<zd>()};
+    }
+    template <typename S>
+    RdPairArgs<S> pair_args(cplx<S>* F, const RdPair* p, const zd* coef, const zd* rtab) const {
+        return RdPairArgs<S>{F,     p,    coef, sh.by, sh.bx, sh.x0, sh.y0, g->nx, g->K(),
+                             rtab, keep.as<uint32_t>(), twx.as<zd>()};
+    }
+    template <typename S>
+    RdInitArgs<S> init_args(cplx<S>* F, const FieldDesc* fd, const zd* amp, const zd* src, bool add) const {
+        return RdInitArgs<S>{F, fd, amp, src, sh.by, sh.bx, sh.x0, sh.y0, g->nx, g->K(), keep.as<uint32_t>(),
+                             twx.as<zd>(), add ? 1 : 0};
+    }
+};
+
+// ---------------------------------------------------------------------------
 // single propagation (bf_propagate)
 // ---------------------------------------------------------------------------
 void propagate_one(bf_ctx* ctx, int kind, const bf_coords* coords, double* E, double dz, double diskR, zd eps,
@@ -1438,6 +1556,10 @@ struct DancerPlan : DancerPlanBase {
         reflect, ph1d, keep_tab;
     int keep_band = 0;  // band class of keep_tab (see prune_class)
     std::unique_ptr<PropEngine<T>> pe;
+    // on the aperture's window (Reduced): column entries [slot][nb 2 R] with the exit fields
+    // last, boundaries [slot][nb (R + 1)], coefficients of the boundaries
+    std::unique_ptr<Reduced> red;
+    DevBuf red_cols, red_pairs, red_coef, red_init;
     DancerOptions opt;
     int nslices;
     std::vector<FieldDesc> fd_host;
@@ -1524,7 +1646,11 @@ struct DancerPlan : DancerPlanBase {
         band_hi = g.ny;
         if (opt.band && amin == 0.0 && (kind == BF_PROP_PROPAGATOR || kind == BF_PROP_NOTILTS))
             aperture_range(g.hY, g.hX, diskR, band_lo, band_hi);
-        const bool qtab = quarter_tables_ok<T>(co, kind);
+        nslices = opt.immediatesum ? 1 : nmax + 1;
+        RdShape rsh;
+        const bool rd = !std::is_same<T, f32pure>::value && nslices == 1 && R >= 2 &&
+                        Reduced::usable(g, kind, amin, nmax, diskR, rsh);
+        const bool qtab = !rd && quarter_tables_ok<T>(co, kind);
         // Frequency batch: what one bounce of a batch touches (the band rows of every
         // field, plus one k-space table per distinct (eps, dz)) is kept near
         // 192 MB, the size of the Infinity Cache; the frequencies are then spread
@@ -1542,8 +1668,9 @@ struct DancerPlan : DancerPlanBase {
             }
             std::sort(keys.begin(), keys.end());
             const size_t ntab = (size_t)(std::unique(keys.begin(), keys.end()) - keys.begin());
-            const size_t touched = sizeof(cplx<S>) * (size_t)(band_hi - band_lo) * g.nx * 2 * R +
-                                   ntab * (qtab ? K / 4 : K) * sizeof(cplx<C>);
+            const size_t touched =
+                rd ? sizeof(cplx<S>) * rsh.field() * 2 * R + ntab * rsh.table() * sizeof(zd)
+                   : sizeof(cplx<S>) * (size_t)(band_hi - band_lo) * g.nx * 2 * R + ntab * (qtab ? K / 4 : K) * sizeof(cplx<C>);
             const size_t budget = (size_t)192 << 20;
             fb = (int)std::max<size_t>(1, budget / std::max<size_t>(touched, 1));
         }
@@ -1553,8 +1680,7 @@ struct DancerPlan : DancerPlanBase {
             fb = (nfreq + nb - 1) / nb;
         }
         freq_batch = fb;
-        nslices = opt.immediatesum ? 1 : nmax + 1;
-        fields.alloc(per * fb);
+        fields.alloc(rd ? sizeof(cplx<S>) * rsh.field() * 2 * R * fb : per * fb);
         if (kind == BF_PROP_MOMENTUM) scratch.alloc(per * fb);
         Eout.alloc(sizeof(zd) * K * nfreq);
         if (nslices > 1) hist.alloc(sizeof(zd) * K * (size_t)nslices * fb);
@@ -1594,6 +1720,18 @@ struct DancerPlan : DancerPlanBase {
         pe.reset(new PropEngine<T>(ctx, &g, kind, diskR, surf.as<zd>()));
         pe->col_tx = opt.col_tx;
         pe->quarter = qtab;
+        if (rd) {
+            red.reset(new Reduced(ctx, &g, rsh, kind, diskR, surf.as<zd>()));
+            std::vector<zd> c4(4 * (size_t)(R + 1));
+            for (int b = 0; b <= R; b++) {
+                c4[4 * b] = r[b];
+                c4[4 * b + 1] = cmk<double>(1.0 - r[b].re, -r[b].im);
+                c4[4 * b + 2] = cmk<double>(1.0 + r[b].re, r[b].im);
+                c4[4 * b + 3] = cmk<double>(-r[b].re, -r[b].im);
+            }
+            red_coef.alloc(sizeof(zd) * c4.size());
+            upload(red_coef.p, c4.data(), sizeof(zd) * c4.size(), s);
+        }
         // aperture bits of the register row pass (thread t of a line holds x = t + (nx/16) m, m < 16)
         if (g.nx >= 16 && g.nx % 16 == 0) {
             const int TT = g.nx / 16;
@@ -1659,7 +1797,151 @@ struct DancerPlan : DancerPlanBase {
         }
     }
 
+    // Replays (or captures, or launches) the bounce loop `loop` of frequency batch f0.
+    template <typename F>
+    void replay(int f0, const void* tab0, const void* tab1, F&& loop) {
+        hipStream_t s = ctx->stream;
+        if (!opt.graph || timing || nmax < 0) {
+            loop();
+            tcollect(nmax + 1);
+            return;
+        }
+        const size_t bi = (size_t)(f0 / fb);
+        if (graphs.size() <= bi) graphs.resize(bi + 1);
+        BatchGraph& bg = graphs[bi];
+        if (bg.exec && (bg.ktab != tab0 || bg.rtab != tab1)) {
+            BF_HIP(hipGraphExecDestroy(bg.exec));
+            bg.exec = nullptr;
+        }
+        if (!bg.exec) {
+            BF_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
+            hipGraph_t gr = nullptr;
+            try {
+                loop();
+            } catch (...) {
+                (void)hipStreamEndCapture(s, &gr);
+                if (gr) (void)hipGraphDestroy(gr);
+                throw;
+            }
+            BF_HIP(hipStreamEndCapture(s, &gr));
+            const hipError_t e = hipGraphInstantiate(&bg.exec, gr, nullptr, nullptr, 0);
+            (void)hipGraphDestroy(gr);
+            BF_HIP(e);
+            bg.ktab = tab0;
+            bg.rtab = tab1;
+        }
+        BF_HIP(hipGraphLaunch(bg.exec, s));
+    }
+
+    // The sweep on the aperture's window: fields [f][region][slot][by][Mx], transformed
+    // along x.  The exit field (region R-1, right-moving) is added to its frequency's sum
+    // before every bounce instead of being propagated; the sums are propagated once.
+    void run_reduced() {
+        hipStream_t s = ctx->stream;
+        const size_t K = g.K(), FK = red->sh.field();
+        cplx<S>* F = fields.as<cplx<S>>();
+        auto grow = [](DevBuf& d, size_t bytes) {
+            if (d.bytes < bytes) d.alloc(bytes);
+        };
+        for (int f0 = 0; f0 < nfreq; f0 += fb) {
+            const int nb = std::min(fb, nfreq - f0);
+            std::vector<RegionParams> regs, last;
+            for (int f = 0; f < nb; f++) {
+                const double lam = 299792458.0 / freqs[f0 + f];
+                for (int i = 0; i < R; i++)
+                    regs.push_back(RegionParams{eps[i], dist[i], tx[i], ty[i], lam, has_surf ? (int64_t)(K * i) : -1});
+                last.push_back(regs.back());
+            }
+            pe->build_tables(regs, true);
+            red->tables(reinterpret_cast<zd*>(pe->ktab.p), pe->ntab);
+            const int nfd = nb * 2 * R, np = nb * (R + 1);
+            std::vector<FieldDesc> init(nfd), col(2 * (size_t)nfd);
+            std::vector<size_t> ord;
+            for (int f = 0; f < nb; f++)
+                for (int q = 0; q < 2 * R; q++) {
+                    FieldDesc& d = init[(size_t)f * 2 * R + q];
+                    d = FieldDesc{(int64_t)(((size_t)f * 2 * R + q) * FK), q, -1, f, 0};
+                    if (opt.reflect && !opt.emit) d.ktab = q == 2 * (R - 1) + 1 ? 0 : -1;
+                    ord.push_back((size_t)f * 2 * R + q);
+                }
+            auto table = [&](size_t q) { return pe->ktab_of[q / 2]; };
+            // blocks that read one table run back to back and find it in L2
+            std::stable_sort(ord.begin(), ord.end(), [&](size_t x, size_t y) { return table(x) < table(y); });
+            std::vector<RdPair> pairs(2 * (size_t)np);
+            for (int rm = 0; rm < 2; rm++) {
+                size_t k = (size_t)rm * nfd, last_k = k + nfd - nb;
+                for (size_t q : ord) {
+                    const bool exit = (int)(q % (2 * R)) == 2 * (R - 1) + rm;
+                    FieldDesc d = init[q];
+                    d.ktab = table(q);
+                    d.rtab = exit ? d.group : -1;
+                    d.pad = exit ? RD_SUM_ONLY : 0;
+                    col[exit ? last_k++ : k++] = d;
+                }
+                for (int f = 0; f < nb; f++)
+                    for (int b = 0; b <= R; b++) {
+                        RdPair& p = pairs[(size_t)rm * np + (size_t)f * (R + 1) + b];
+                        p = RdPair{0, 0, -1, -1, b, 0};
+                        auto field = [&](int reg, int slot) { return (int64_t)((((size_t)f * R + reg) * 2 + slot) * FK); };
+                        auto rt = [&](int reg) { return pe->rtab_of.empty() ? -1 : pe->rtab_of[(size_t)f * R + reg]; };
+                        if (b > 0) {
+                            p.off0 = field(b - 1, rm);
+                            p.rt0 = rt(b - 1);
+                            p.flags |= b < R ? RP_LOAD0 | RP_STORE0 : RP_ZERO0;  // r = 0 at the exit boundary
+                        }
+                        if (b < R) {
+                            p.off1 = field(b, 1 - rm);
+                            p.rt1 = rt(b);
+                            p.flags |= RP_LOAD1 | RP_STORE1;
+                        }
+                    }
+            }
+            grow(red_init, sizeof(FieldDesc) * init.size());
+            grow(red_cols, sizeof(FieldDesc) * 2 * (size_t)fb * 2 * R);
+            grow(red_pairs, sizeof(RdPair) * 2 * (size_t)fb * (R + 1));
+            upload(red_init.p, init.data(), sizeof(FieldDesc) * init.size(), s);
+            upload(red_cols.p, col.data(), sizeof(FieldDesc) * col.size(), s);
+            upload(red_pairs.p, pairs.data(), sizeof(RdPair) * pairs.size(), s);
+            const zd* src = opt.emit ? emit.as<zd>() : opt.reflect ? reflect.as<zd>() : nullptr;
+            rd_init(red->sh, red->template init_args<S>(F, red_init.as<FieldDesc>(), src ? nullptr : ax.as<zd>(), src, false),
+                    nfd, s);
+            red->clear_sums(nb);
+            const zd* rt = pe->has_rtab() ? reinterpret_cast<const zd*>(pe->rtab.p) : nullptr;
+            auto loop = [&] {
+                int rm = 0;
+                for (int n = 0; n <= nmax; n++) {
+                    const FieldDesc* cd = red_cols.as<FieldDesc>() + (size_t)rm * nfd;
+                    tmark(n, 1, 0);
+                    if (n < nmax)
+                        rd_cols(red->sh, red->template col_args<S>(F, cd), nfd, s);
+                    else
+                        rd_cols(red->sh, red->template col_args<S>(F, cd + nfd - nb), nb, s);
+                    tmark(n, 1, 1);
+                    tmark(n, 0, 0);
+                    if (n < nmax)
+                        rd_pairs(red->sh, red->template pair_args<S>(F, red_pairs.as<RdPair>() + (size_t)rm * np,
+                                                                      red_coef.as<zd>(), rt), np, s);
+                    tmark(n, 0, 1);
+                    rm = 1 - rm;
+                }
+            };
+            replay(f0, red->tabs.p, rt, loop);
+            zd* eout = Eout.as<zd>() + (size_t)f0 * K;
+            red->propagate_sums(0, last, eout);
+            hipLaunchKernelGGL(k_power, dim3(nb), dim3(1024), 0, s, eout, K, power.as<double>() + f0);
+            BF_CHECK_LAUNCH();
+        }
+        std::vector<int> done(nfreq, nmax + 1);
+        upload(count.p, done.data(), sizeof(int) * nfreq, s);
+    }
+
     void run() override {
+        if constexpr (!std::is_same<T, f32pure>::value) {
+            if (red) {
+                run_reduced();
+                return;
+            }
+        }
         hipStream_t s = ctx->stream;
         const size_t K = g.K();
         const bool fused = (kind == BF_PROP_PROPAGATOR || kind == BF_PROP_NOTILTS);
@@ -1741,36 +2023,7 @@ struct DancerPlan : DancerPlanBase {
             int rm = 0;
             if (fused) {
                 pe->rows(fields.as<cplx<S>>(), fd, nf, RF_MASK | RF_FWD, active.as<int>());
-                if (opt.graph && !timing && nmax >= 0) {
-                    const size_t bi = (size_t)(f0 / fb);
-                    if (graphs.size() <= bi) graphs.resize(bi + 1);
-                    BatchGraph& bg = graphs[bi];
-                    if (bg.exec && (bg.ktab != pe->ktab.p || bg.rtab != pe->rtab.p)) {
-                        BF_HIP(hipGraphExecDestroy(bg.exec));
-                        bg.exec = nullptr;
-                    }
-                    if (!bg.exec) {
-                        BF_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
-                        hipGraph_t gr = nullptr;
-                        try {
-                            bounce_loop(f0, nb, eo_target);
-                        } catch (...) {
-                            (void)hipStreamEndCapture(s, &gr);
-                            if (gr) (void)hipGraphDestroy(gr);
-                            throw;
-                        }
-                        BF_HIP(hipStreamEndCapture(s, &gr));
-                        const hipError_t e = hipGraphInstantiate(&bg.exec, gr, nullptr, nullptr, 0);
-                        (void)hipGraphDestroy(gr);
-                        BF_HIP(e);
-                        bg.ktab = pe->ktab.p;
-                        bg.rtab = pe->rtab.p;
-                    }
-                    BF_HIP(hipGraphLaunch(bg.exec, s));
-                } else {
-                    bounce_loop(f0, nb, eo_target);
-                    tcollect(nmax + 1);
-                }
+                replay(f0, pe->ktab.p, pe->rtab.p, [&] { bounce_loop(f0, nb, eo_target); });
             } else {
                 for (int n = 0; n <= nmax; n++) {
                     pe->propagate(fields.as<cplx<S>>(), fd, nf, ph1d.as<zd>(), scratch.as<cplx<S>>(),

@@ -192,6 +192,7 @@ struct EngineOptions {
     int prune = 1;            // band-pruned register transforms
     int qtab = 1;             // quarter k-space tables for complex64 fields
     int band = 1;             // skip the rows the aperture zeroes
+    int reduced = 1;          // bounce solvers on the aperture's window (amin 0, summed output)
     int chfuse = 1;           // cheerleader: pair steps fused with their boundary update
     int chxf = 1;             // cheerleader: pair steps store the next masked row transform
     int chwave = 1;           // cheerleader: wavefront order when amin is 0

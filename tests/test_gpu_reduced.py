@@ -1,0 +1,95 @@
+"""The bounce solvers on the aperture's window (circular convolutions of 16 R points per
+line) against the transforms of the whole grid: every radix, windows at the edge of a
+radix and of the grid, rectangular grids, tilts and surfaces, given emission and
+reflection, batches of frequencies, replayed graphs."""
+import numpy as np
+import pytest
+
+import BoostFractor as B
+from BoostFractor import workloads as W
+from helpers import DISKR, rel
+
+pytestmark = pytest.mark.gpu
+# whole-grid and windowed transforms round differently by ~1e-15 per bounce; fields stored
+# in complex64 round at 6e-8 of their maximum per pass
+TOL = {"fp64": 1e-12, "mixed": 2e-6}
+
+
+def _both(fn):
+    out = []
+    for on in (1, 0):
+        with B.context().options(reduced=on):
+            out.append(fn())
+    return out
+
+
+def _grid(nx, ny, shift=0):
+    def axis(n):
+        return (np.arange(n) - n // 2 + shift) / 128.0
+    X, Y = axis(nx), axis(ny)
+    k = lambda v: (np.arange(len(v)) - (len(v) - 1) / 2.0) * 2 * np.pi / (len(v) / 128.0)  # noqa: E731
+    return B.CoordinateSystem(X, Y, k(X), k(Y))
+
+
+def _booster(c, rough, seed):
+    sb = W.rough_booster(c, ndisk=2, seed=seed) if rough else W.booster(c, ndisk=2, seed=seed)
+    return sb
+
+
+# radius in samples of 1/128 m: bands of 2 r - 1 .. 2 r + 1 samples, radices 4, 5, 6, 8, 10, 12, 16, 20
+@pytest.mark.parametrize("radius", [3.2, 16.0, 16.6, 20.4, 24.0, 24.3, 32.4, 40.3, 48.5, 63.9, 64.2, 79.9])
+@pytest.mark.parametrize("prec", ["fp64", "mixed"])
+def test_dancer_on_every_radix(radius, prec):
+    n = 128 if radius < 32 else 256 if radius < 64 else 512
+    c = _grid(n, n)
+    sb = _booster(c, False, 11)
+    R = radius / 128.0
+    a, b = _both(lambda: B.dancer(0, 9, sb, c, f=[19.8e9, 20.2e9], diskR=R, precision=prec))
+    assert np.any(b != 0) and rel(a, b) < TOL[prec]
+
+
+@pytest.mark.parametrize("nx,ny,shift", [(128, 256, 0), (101, 130, 0), (150, 100, 0), (256, 128, 30), (200, 120, -58),
+                                         (97, 512, 5)])
+@pytest.mark.parametrize("prec", ["fp64", "mixed"])
+def test_dancer_on_other_grids_and_windows(nx, ny, shift, prec):
+    """rectangular grids; windows off the centre, cut by the grid's edge"""
+    c = _grid(nx, ny, shift)
+    sb = _booster(c, True, 12)
+    refl = np.exp(-(c.X[None] ** 2 + c.Y[:, None] ** 2) / 0.1 ** 2) * np.exp(3j * c.X[None])
+    rng = np.random.default_rng(3)
+    emit = rng.standard_normal((len(sb.distance) - 1, 2, ny, nx)) + 0j
+    for kw in ({}, {"reflect": refl}, {"emit": emit}):
+        a, b = _both(lambda: B.dancer(0, 8, sb, c, f=[20e9], diskR=DISKR, precision=prec, **kw))
+        assert np.any(b != 0) and rel(a, b) < TOL[prec]
+    a, b = _both(lambda: B.dancer(0, 8, sb, c, f=20e9, prop=B.propagatorNoTilts, diskR=DISKR, precision=prec))
+    assert rel(a, b) < TOL[prec]
+
+
+@pytest.mark.parametrize("prec", ["fp64", "mixed"])
+def test_dancer_plans_batches_and_graphs(prec):
+    c = _grid(128, 128)
+    sb = _booster(c, True, 13)
+    f = np.linspace(19.5e9, 20.5e9, 7)
+    want = B.dancer(0, 10, sb, c, f=f, diskR=DISKR, precision=prec)
+    for graph in (0, 1):
+        with B.context().options(graph=graph):
+            plan = B.DancerPlan(0, 10, sb, c, f, diskR=DISKR, precision=prec, freq_batch=3)
+            for _ in range(3):
+                plan.run()
+                B.dancer(0, 8, sb, c, f=20e9, diskR=DISKR)  # eager work on the same stream in between
+                E, power = plan.fetch()
+                assert np.array_equal(E, want)
+                assert np.allclose(power, np.sum(np.abs(want) ** 2, axis=(1, 2)), rtol=1e-12)
+            plan.close()
+
+
+def test_history_amin_and_short_runs_keep_the_whole_grid():
+    c = _grid(128, 128)
+    sb = _booster(c, False, 14)
+    for kw in ({"returnsum": False, "immediatesum": False}, {"returnsum": True, "immediatesum": False}):
+        a, b = _both(lambda: B.dancer(0, 9, sb, c, f=20e9, diskR=DISKR, **kw))
+        assert np.array_equal(a, b)
+    a, b = _both(lambda: B.dancer(0.05, 30, sb, c, f=20e9, diskR=DISKR))
+    assert np.array_equal(a, b)
+    a, b = _both(lambda: B.dancer(0, 3, sb, c, f=20e9, diskR=DISKR))
+    assert np.array_equal(a, b)
