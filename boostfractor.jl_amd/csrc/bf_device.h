@@ -148,30 +148,31 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t buf_rsrc(const void* base, uin
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, (int)bytes, 0x00020000);
 }
 
+// (uni: a wave-uniform part of the offset, added by the instruction)
 template <typename S>
-__device__ __forceinline__ cplx<S> buf_load(__amdgpu_buffer_rsrc_t r, uint32_t off);
+__device__ __forceinline__ cplx<S> buf_load(__amdgpu_buffer_rsrc_t r, uint32_t off, uint32_t uni = 0);
 template <>
-__device__ __forceinline__ cplx<float> buf_load<float>(__amdgpu_buffer_rsrc_t r, uint32_t off) {
-    const auto v = __builtin_amdgcn_raw_buffer_load_b64(r, (int)off, 0, 0);
+__device__ __forceinline__ cplx<float> buf_load<float>(__amdgpu_buffer_rsrc_t r, uint32_t off, uint32_t uni) {
+    const auto v = __builtin_amdgcn_raw_buffer_load_b64(r, (int)off, (int)uni, 0);
     return cmk<float>(__uint_as_float(v[0]), __uint_as_float(v[1]));
 }
 template <>
-__device__ __forceinline__ cplx<double> buf_load<double>(__amdgpu_buffer_rsrc_t r, uint32_t off) {
-    const auto v = __builtin_amdgcn_raw_buffer_load_b128(r, (int)off, 0, 0);
+__device__ __forceinline__ cplx<double> buf_load<double>(__amdgpu_buffer_rsrc_t r, uint32_t off, uint32_t uni) {
+    const auto v = __builtin_amdgcn_raw_buffer_load_b128(r, (int)off, (int)uni, 0);
     return cmk<double>(__hiloint2double((int)v[1], (int)v[0]), __hiloint2double((int)v[3], (int)v[2]));
 }
 
 template <typename S>
-__device__ __forceinline__ void buf_store(__amdgpu_buffer_rsrc_t r, uint32_t off, cplx<S> a);
+__device__ __forceinline__ void buf_store(__amdgpu_buffer_rsrc_t r, uint32_t off, cplx<S> a, uint32_t uni = 0);
 template <>
-__device__ __forceinline__ void buf_store<float>(__amdgpu_buffer_rsrc_t r, uint32_t off, cplx<float> a) {
+__device__ __forceinline__ void buf_store<float>(__amdgpu_buffer_rsrc_t r, uint32_t off, cplx<float> a, uint32_t uni) {
     unsigned int v __attribute__((__vector_size__(8)));
     v[0] = __float_as_uint(a.re);
     v[1] = __float_as_uint(a.im);
-    __builtin_amdgcn_raw_buffer_store_b64(v, r, (int)off, 0, 0);
+    __builtin_amdgcn_raw_buffer_store_b64(v, r, (int)off, (int)uni, 0);
 }
 template <>
-__device__ __forceinline__ void buf_store<double>(__amdgpu_buffer_rsrc_t r, uint32_t off, cplx<double> a) {
+__device__ __forceinline__ void buf_store<double>(__amdgpu_buffer_rsrc_t r, uint32_t off, cplx<double> a, uint32_t uni) {
     unsigned int v __attribute__((__vector_size__(16)));
     const unsigned long long re = (unsigned long long)__double_as_longlong(a.re);
     const unsigned long long im = (unsigned long long)__double_as_longlong(a.im);
@@ -179,7 +180,7 @@ __device__ __forceinline__ void buf_store<double>(__amdgpu_buffer_rsrc_t r, uint
     v[1] = (unsigned int)(re >> 32);
     v[2] = (unsigned int)im;
     v[3] = (unsigned int)(im >> 32);
-    __builtin_amdgcn_raw_buffer_store_b128(v, r, (int)off, 0, 0);
+    __builtin_amdgcn_raw_buffer_store_b128(v, r, (int)off, (int)uni, 0);
 }
 
 // ---------------------------------------------------------------------------

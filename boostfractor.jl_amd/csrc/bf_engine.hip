@@ -860,9 +860,17 @@ void download(void* dst, const void* src, size_t bytes, hipStream_t s) {
     if (bytes) BF_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s));
 }
 
-void Grid::upload(const bf_coords* c, hipStream_t s) {
+void Grid::host(const bf_coords* c) {
     nx = c->nx;
     ny = c->ny;
+    hX.assign(c->X, c->X + nx);
+    hY.assign(c->Y, c->Y + ny);
+    hkX.assign(c->kX, c->kX + nx);
+    hkY.assign(c->kY, c->kY + ny);
+}
+
+void Grid::upload(const bf_coords* c, hipStream_t s) {
+    host(c);
     const int len[4] = {nx, ny, nx, ny};
     const double* src[4] = {c->X, c->Y, c->kX, c->kY};
     View* view[4] = {&X, &Y, &kX, &kY};
@@ -876,10 +884,6 @@ void Grid::upload(const bf_coords* c, hipStream_t s) {
         view[q]->p = d;
         d += len[q];
     }
-    hX.assign(c->X, c->X + nx);
-    hY.assign(c->Y, c->Y + ny);
-    hkX.assign(c->kX, c->kX + nx);
-    hkY.assign(c->kY, c->kY + ny);
 }
 
 template <typename T>
@@ -1298,6 +1302,15 @@ static zd phase_1d(zd eps, double lambda, double dz) {
     return cexp_j(cmk<double>(dz * e.re, dz * e.im));
 }
 
+// a mirror-symmetric k range: k[j] = -k[n-1-j] up to rounding
+static bool k_mirrored(const double* k, int len) {
+    double mx = 0.0;
+    for (int j = 0; j < len; j++) mx = std::max(mx, std::fabs(k[j]));
+    for (int j = 0; j < len; j++)
+        if (!(std::fabs(k[j] + k[len - 1 - j]) <= 1e-12 * mx)) return false;
+    return true;
+}
+
 // ---------------------------------------------------------------------------
 // propagation on the aperture's window (bf_reduced.h)
 // ---------------------------------------------------------------------------
@@ -1314,9 +1327,10 @@ struct Reduced {
     std::unique_ptr<PropEngine<double>> pn, pm;  // whole grid; reduced grid
     DevBuf tabs, keep, twx, twy, sum, fdn, fdm, fdout;
 
-    // The window of the grid's aperture, when the reduced convolution is at most 3/4 of the
-    // grid (a power of two) or no larger than it (other sizes, whose own lines take 2 n^2
-    // flop on the matrix cores): below that the smaller lines win at every size measured.
+    // The window of the grid's aperture, when the reduced convolution is at most 3/4 of the grid (a power
+    // of two) or no larger than it (other sizes, whose own lines take 2 n^2 flop on the matrix cores).
+    // Measured at 0.39 of 256^2 and 512^2 (1.5 and 2.2 times faster) and 0.63 of 101^2 (2.5 times); 192 of
+    // 256 points a line, 0.56, is the next larger shape below the grid's own.
     static bool shape(const Grid& g, double diskR, RdShape& sh) {
         int lo, hi;
         aperture_range(g.hY, g.hX, diskR, lo, hi);
@@ -1329,8 +1343,11 @@ struct Reduced {
         sh.Ry = rd_radix(sh.by);
         sh.Rx = rd_radix(sh.bx);
         if (!sh.Ry || !sh.Rx) return false;
+        sh.quarter = k_mirrored(g.hkX.data(), g.nx) && k_mirrored(g.hkY.data(), g.ny);
+        sh.ex = sh.quarter && g.nx % 2 == 0 ? 1.0 / g.nx : 0.0;
+        sh.ey = sh.quarter && g.ny % 2 == 0 ? 1.0 / g.ny : 0.0;
         const bool pow2 = !dft_length(g.nx) && !dft_length(g.ny);
-        return pow2 ? 4 * sh.table() <= 3 * g.K() : sh.table() <= g.K();
+        return pow2 ? 4 * sh.points() <= 3 * g.K() : sh.points() <= g.K();
     }
     static bool usable(const Grid& g, int kind, double amin, int nmax, double diskR, RdShape& sh) {
         return opts().reduced && use_reg_fft() && amin == 0.0 && nmax + 1 >= MIN_BOUNCES &&
@@ -1364,7 +1381,7 @@ struct Reduced {
         std::vector<FieldDesc> a(ntab), b(ntab);
         for (int j = 0; j < ntab; j++) {
             a[j] = FieldDesc{(int64_t)j * (int64_t)K, -1, -1, 0, 0};
-            b[j] = FieldDesc{(int64_t)j * (int64_t)sh.table(), -1, -1, 0, 0};
+            b[j] = FieldDesc{(int64_t)j * (int64_t)sh.points(), -1, -1, 0, 0};
         }
         auto put = [&](DevBuf& d, const std::vector<FieldDesc>& v) {
             if (d.bytes < sizeof(FieldDesc) * v.size()) d.alloc(sizeof(FieldDesc) * v.size());
@@ -1373,24 +1390,29 @@ struct Reduced {
         put(fdn, a);
         put(fdm, b);
         if (tabs.bytes < sizeof(zd) * sh.table() * ntab) tabs.alloc(sizeof(zd) * sh.table() * ntab);
+        DevBuf full;
+        if (sh.quarter) full.alloc(sizeof(zd) * sh.points() * ntab);
+        zd* M = sh.quarter ? full.as<zd>() : tabs.as<zd>();
         pn->rows(T, fdn.as<FieldDesc>(), ntab, RF_INV, nullptr);
         pn->cols(T, T, fdn.as<FieldDesc>(), ntab, CF_INV, nullptr);
-        rd_crop(sh, T, g->nx, g->ny, ntab, tabs.as<zd>(), ctx->stream);
-        pm->rows(tabs.as<zd>(), fdm.as<FieldDesc>(), ntab, RF_FWD, nullptr);
-        pm->cols(tabs.as<zd>(), tabs.as<zd>(), fdm.as<FieldDesc>(), ntab, CF_FWD, nullptr);
+        rd_crop(sh, T, g->nx, g->ny, ntab, M, ctx->stream);
+        pm->rows(M, fdm.as<FieldDesc>(), ntab, RF_FWD, nullptr);
+        pm->cols(M, M, fdm.as<FieldDesc>(), ntab, CF_FWD, nullptr);
+        if (sh.quarter) rd_quarter(sh, M, ntab, tabs.as<zd>(), ctx->stream);
     }
     void clear_sums(int n) {
         const size_t bytes = sizeof(zd) * sh.field() * n;
         if (sum.bytes < bytes) sum.alloc(bytes);
         BF_HIP(hipMemsetAsync(sum.p, 0, bytes, ctx->stream));
     }
-    // out[j] = propagation of sum slot0 + j by region regs[j] on the whole grid
-    void propagate_sums(int slot0, const std::vector<RegionParams>& regs, zd* out) {
+    // out[j] = propagation of sum slot0 + j (pair: of complex64 fields) by region regs[j] on the whole grid
+    void propagate_sums(int slot0, const std::vector<RegionParams>& regs, bool pair, zd* out) {
         const size_t K = g->K();
         const int n = (int)regs.size();
         BF_HIP(hipMemsetAsync(out, 0, sizeof(zd) * K * n, ctx->stream));
-        RdFinalArgs fa{sum.as<zd>() + (size_t)slot0 * sh.field(), out, sh.by, sh.bx, sh.x0, sh.y0, g->nx, K, twx.as<zd>()};
-        rd_final(sh, fa, n, ctx->stream);
+        RdFinalArgs fa{sum.as<zd>() + (size_t)slot0 * sh.field(), out, sh.by, sh.bx, sh.x0, sh.y0, g->nx, K, twx.as<zd>(),
+                       sh.ex, sh.ey};
+        rd_final(sh, fa, n, pair, ctx->stream);
         pn->build_tables(regs);
         std::vector<FieldDesc> fd(n);
         for (int j = 0; j < n; j++)
@@ -1401,7 +1423,7 @@ struct Reduced {
     }
     template <typename S>
     RdColArgs<S> col_args(cplx<S>* F, const FieldDesc* fd) const {
-        return RdColArgs<S>{F, fd, sh.Mx(), sh.by, tabs.as<zd>(), sum.as<zd>(), twy.as<zd>()};
+        return RdColArgs<S>{F, fd, sh.Rx, sh.by, tabs.as<zd>(), sh.quarter ? 1 : 0, sum.as<zd>(), twy.as<zd>()};
     }
     template <typename S>
     RdPairArgs<S> pair_args(cplx<S>* F, const RdPair* p, const zd* coef, const zd* rtab) const {
@@ -1411,7 +1433,7 @@ struct Reduced {
     template <typename S>
     RdInitArgs<S> init_args(cplx<S>* F, const FieldDesc* fd, const zd* amp, const zd* src, bool add) const {
         return RdInitArgs<S>{F, fd, amp, src, sh.by, sh.bx, sh.x0, sh.y0, g->nx, g->K(), keep.as<uint32_t>(),
-                             twx.as<zd>(), add ? 1 : 0};
+                             twx.as<zd>(), sh.ex, sh.ey, add ? 1 : 0};
     }
 };
 
@@ -1520,16 +1542,9 @@ void dance_intro_dev(bf_ctx* ctx, const bf_coords* coords, int nd, const double*
 template <typename T>
 static bool quarter_tables_ok(const bf_coords* co, int kind) {
     const int n = co->nx;
-    auto mirrored = [](const double* k, int len) {
-        double mx = 0.0;
-        for (int j = 0; j < len; j++) mx = std::max(mx, std::fabs(k[j]));
-        for (int j = 0; j < len; j++)
-            if (!(std::fabs(k[j] + k[len - 1 - j]) <= 1e-12 * mx)) return false;
-        return true;
-    };
     return !std::is_same<T, double>::value && opts().qtab && use_reg_fft() &&
            (kind == BF_PROP_PROPAGATOR || kind == BF_PROP_NOTILTS) && co->nx == co->ny && n >= 16 && n <= 1024 &&
-           (n & (n - 1)) == 0 && mirrored(co->kX, co->nx) && mirrored(co->kY, co->ny);
+           (n & (n - 1)) == 0 && k_mirrored(co->kX, co->nx) && k_mirrored(co->kY, co->ny);
 }
 
 template <typename T>
@@ -1648,7 +1663,7 @@ struct DancerPlan : DancerPlanBase {
             aperture_range(g.hY, g.hX, diskR, band_lo, band_hi);
         nslices = opt.immediatesum ? 1 : nmax + 1;
         RdShape rsh;
-        const bool rd = !std::is_same<T, f32pure>::value && nslices == 1 && R >= 2 &&
+        const bool rd = std::is_same<T, double>::value && nslices == 1 && R >= 2 &&
                         Reduced::usable(g, kind, amin, nmax, diskR, rsh);
         const bool qtab = !rd && quarter_tables_ok<T>(co, kind);
         // Frequency batch: what one bounce of a batch touches (the band rows of every
@@ -1927,7 +1942,7 @@ struct DancerPlan : DancerPlanBase {
             };
             replay(f0, red->tabs.p, rt, loop);
             zd* eout = Eout.as<zd>() + (size_t)f0 * K;
-            red->propagate_sums(0, last, eout);
+            red->propagate_sums(0, last, false, eout);
             hipLaunchKernelGGL(k_power, dim3(nb), dim3(1024), 0, s, eout, K, power.as<double>() + f0);
             BF_CHECK_LAUNCH();
         }
@@ -1936,7 +1951,7 @@ struct DancerPlan : DancerPlanBase {
     }
 
     void run() override {
-        if constexpr (!std::is_same<T, f32pure>::value) {
+        if constexpr (std::is_same<T, double>::value) {
             if (red) {
                 run_reduced();
                 return;
@@ -2083,6 +2098,15 @@ struct DancerPlan : DancerPlanBase {
 static DancerPlanBase* make_dancer_plan_fixed(bf_ctx* ctx, const bf_setup* st, const bf_coords* co, double amin,
                                               int nmax, const double* fr, int nfr, int kind, double diskR,
                                               int precision, const DancerOptions& o) {
+    // On the window mixed precision keeps complex128 fields too: complex64 ones are 12% faster (the 20-disk
+    // booster, 256^2, 20 frequencies: 46.7 against 53.1 ms; 512^2, 4: 21.2 against 23.8) but round the
+    // emitted fields 0.7 to 1.35 times as far as the whole grid's mixed passes and their power up to twice.
+    if (precision == BF_PREC_MIXED && st->nreg > 2 && (o.immediatesum || nmax == 0)) {
+        Grid g;
+        g.host(co);
+        RdShape sh;
+        if (Reduced::usable(g, kind, amin, nmax, diskR, sh)) precision = BF_PREC_FP64;
+    }
     if (precision == BF_PREC_MIXED) {
         auto* p = new DancerPlan<float>();
         try { p->init(ctx, st, co, amin, nmax, fr, nfr, kind, diskR, o); } catch (...) { delete p; throw; }
@@ -2381,6 +2405,213 @@ __global__ void k_amax_fields(const cplx<typename Storage<T>::type>* F, size_t n
     if ((threadIdx.x & 63) == 0 && m > 0.0) atomic_max_pos(amax + f, m);
 }
 
+
+// out = b0 base0 + b1 base1 + t out on nf whole-grid fields: what the summed propagations
+// of a cheerleader leave at an end, and the emission that never propagates.  Without base
+// fields the emission is the constant amplitude b0 on the aperture (edge included).
+__global__ void k_ch_output(zd* out, size_t K, int nx, const zd* base0, const zd* base1, zd b0, zd b1, zd t,
+                            const double* __restrict__ X, const double* __restrict__ Y, double R2, int mask) {
+    zd* o = out + (size_t)blockIdx.y * K;
+    for (size_t p = (size_t)blockIdx.x * blockDim.x + threadIdx.x; p < K; p += (size_t)gridDim.x * blockDim.x) {
+        zd v = cmul(t, o[p]);
+        if (mask) {
+            const double x = X[p % nx], y = Y[p / nx];
+            if (!(x * x + y * y > R2)) v = cadd(v, b0);
+        } else {
+            if (base0) v = cadd(v, cmul(b0, base0[p]));
+            if (base1) v = cadd(v, cmul(b1, base1[p]));
+        }
+        o[p] = v;
+    }
+}
+
+// The sweep on the aperture's window (bf_reduced.h), amin = 0: the interior fields
+// F[1..Nd-2] are only read by masked propagations, so they live on the window,
+// transformed along x; the outputs F[0] and F[Nd-1] only collect propagated fields, so
+// the fields that reach them are summed and propagated once.  Step j of iteration n
+// (j = 0 first region, 1..Nd-3 pair (j, j+1), Nd-2 last region) runs at time 2n + j as
+// in the whole-grid sweep; a time is two launches (columns, then boundaries).
+template <typename T>
+static void cheerleader_reduced(bf_ctx* ctx, const Grid& g, const RdShape& sh, const bf_setup* st, int nmax,
+                                const double* fr, int nfr, int kind, const double* emit_h, const double* reflect_h,
+                                double diskR, const zd* surfaces, const std::vector<zd>& rl, const std::vector<zd>& rr,
+                                const std::vector<zd>& tl, const std::vector<zd>& tr, double* out_right,
+                                double* out_left) {
+    using S = typename Storage<T>::type;
+    hipStream_t s = ctx->stream;
+    const size_t K = g.K(), FK = sh.field();
+    const int Nd = st->nreg, NI = Nd - 2;
+    const zd* eps = reinterpret_cast<const zd*>(st->eps);
+    const zd* r = reinterpret_cast<const zd*>(st->r);
+    // frequencies per batch: whole-grid tables of a batch within 2 GB, fields of a launch within grid.y
+    int fb = (int)std::max<size_t>(1, ((size_t)2 << 30) / (sizeof(zd) * K * (size_t)NI));
+    fb = std::max(1, std::min({fb, nfr, 256, 65535 / (Nd + 2)}));
+    const int sides = out_left ? 2 : 1;
+    DevBuf F(sizeof(cplx<S>) * FK * NI * fb), out(sizeof(zd) * K * fb), dcoef(sizeof(zd) * 4 * Nd), damp, dsrc, dinit, dlist, dpair;
+    PropEngine<T> pe(ctx, &g, kind, diskR, surfaces);
+    Reduced red(ctx, &g, sh, kind, diskR, surfaces);
+    std::vector<zd> cf(4 * (size_t)Nd);
+    for (int i = 0; i < Nd; i++) {
+        cf[4 * i] = rr[i];
+        cf[4 * i + 1] = tl[i];
+        cf[4 * i + 2] = tr[i];
+        cf[4 * i + 3] = rl[i];
+    }
+    upload(dcoef.p, cf.data(), sizeof(zd) * cf.size(), s);
+    // sources: right- and left-moving emission of region i (0..Nd-1) at 2 i, 2 i + 1 (constant
+    // amplitudes or fields); the last interior region's left-moving one with what the last
+    // region's emission transmits into it at 2 Nd
+    std::vector<zd> amp(2 * (size_t)Nd + 1, cmk<double>(0, 0)), extra;
+    if (emit_h || reflect_h) {
+        extra.resize(K);
+        const zd* last = reinterpret_cast<const zd*>(emit_h ? emit_h + 2 * K * (2 * (size_t)(Nd - 1) + 1) : reflect_h);
+        const zd* own = emit_h ? reinterpret_cast<const zd*>(emit_h) + K * (2 * (size_t)(Nd - 2) + 1) : nullptr;
+        for (size_t p = 0; p < K; p++) {
+            extra[p] = cmul(tl[Nd - 2], last[p]);
+            if (own) extra[p] = cadd(own[p], extra[p]);
+        }
+        dsrc.alloc(sizeof(zd) * K * (emit_h ? 2 * (size_t)Nd + 1 : 2));
+        if (emit_h) {
+            upload(dsrc.p, emit_h, sizeof(zd) * K * 2 * Nd, s);
+            upload(dsrc.as<zd>() + K * 2 * Nd, extra.data(), sizeof(zd) * K, s);
+        } else {
+            upload(dsrc.p, extra.data(), sizeof(zd) * K, s);
+            upload(dsrc.as<zd>() + K, reflect_h, sizeof(zd) * K, s);
+        }
+    } else {
+        // dance_intro on the copy with distance[2:end], eps[2:end] and the original r (:262-267)
+        const std::vector<zd> a = dance_intro_amplitudes(Nd - 1, eps + 1, r[0]);
+        for (size_t q = 0; q < a.size(); q++) amp[2 + q] = a[q];
+        amp[2 * Nd] = cadd(amp[2 * (Nd - 2) + 1], cmul(tl[Nd - 2], amp[2 * (Nd - 1) + 1]));
+        damp.alloc(sizeof(zd) * amp.size());
+        upload(damp.p, amp.data(), sizeof(zd) * amp.size(), s);
+    }
+    const zd* src = dsrc.p ? dsrc.as<zd>() : nullptr;
+    for (int f0 = 0; f0 < nfr; f0 += fb) {
+        const int nb = std::min(fb, nfr - f0);
+        std::vector<RegionParams> regs, first, last;
+        for (int f = 0; f < nb; f++) {
+            const double lam = 299792458.0 / fr[f0 + f];
+            for (int i = 1; i <= NI; i++)
+                regs.push_back(RegionParams{eps[i], st->distance[i], st->tilt_x[i], st->tilt_y[i], lam,
+                                            surfaces ? (int64_t)(K * i) : -1});
+            first.push_back(regs[regs.size() - NI]);
+            last.push_back(regs.back());
+        }
+        pe.build_tables(regs, true);
+        red.tables(reinterpret_cast<zd*>(pe.ktab.p), pe.ntab);
+        red.clear_sums(sides * nb);
+        const zd* rt = pe.has_rtab() ? reinterpret_cast<const zd*>(pe.rtab.p) : nullptr;
+        cplx<S>* Fp = F.as<cplx<S>>();
+        auto reg = [&](int f, int i) { return (size_t)f * NI + i - 1; };
+        auto off = [&](int f, int i) { return (int64_t)(reg(f, i) * FK); };
+        auto rtab = [&](int f, int i) { return pe.rtab_of.empty() ? -1 : pe.rtab_of[reg(f, i)]; };
+        auto col = [&](std::vector<FieldDesc>& v, int f, int i, int slot) {
+            v.push_back(FieldDesc{off(f, i), pe.ktab_of[reg(f, i)], slot, f, 0});
+        };
+        // boundary j of frequency f; the fields it updates and how
+        auto bound = [&](std::vector<RdPair>& v, int f, int j, int flags) {
+            RdPair p{0, 0, -1, -1, j, flags};
+            if (j >= 1) {
+                p.off0 = off(f, j);
+                p.rt0 = rtab(f, j);
+            }
+            if (j + 1 <= NI) {
+                p.off1 = off(f, j + 1);
+                p.rt1 = rtab(f, j + 1);
+            }
+            v.push_back(p);
+        };
+        // entries of every launch: [range of columns, range of boundaries]
+        struct Step {
+            size_t c, p;
+            int nc, np;
+        };
+        std::vector<FieldDesc> cl;
+        std::vector<RdPair> pl;
+        std::vector<Step> prologue, steps;
+        auto close = [&](size_t c, size_t p) { return Step{c, p, (int)(cl.size() - c), (int)(pl.size() - p)}; };
+        if (emit_h || !reflect_h)  // (:281-286; nothing moves right in a reflection before the loop)
+            for (int i = 1; i <= NI; i++) {
+                const size_t c = cl.size(), p = pl.size();
+                for (int f = 0; f < nb; f++) {
+                    col(cl, f, i, i == NI ? f : -1);
+                    bound(pl, f, i, RP_LOAD0 | RP_STORE0 | (i < NI ? RP_ADD1 : 0));
+                }
+                prologue.push_back(close(c, p));
+            }
+        std::map<std::pair<int, int>, Step> seen;
+        for (int tau = 0; tau <= 2 * nmax + Nd - 2; tau++) {
+            int jlo = std::max(0, tau - 2 * nmax), jhi = std::min(Nd - 2, tau);
+            if ((tau - jlo) & 1) jlo++;
+            if ((tau - jhi) & 1) jhi--;
+            if (jlo > jhi) continue;
+            auto it = seen.find({jlo, jhi});
+            if (it == seen.end()) {
+                const size_t c = cl.size(), p = pl.size();
+                for (int j = jlo; j <= jhi; j += 2)
+                    for (int f = 0; f < nb; f++) {
+                        if (j >= 1) col(cl, f, j, j == NI ? f : -1);
+                        if (j + 1 <= NI) col(cl, f, j + 1, j == 0 && out_left ? nb + f : -1);
+                    }
+                // the boundaries in descending j: a launch reads first what the one before wrote last
+                for (int j = jhi; j >= jlo; j -= 2)
+                    for (int f = 0; f < nb; f++)
+                        bound(pl, f, j, (j >= 1 ? RP_LOAD0 | RP_STORE0 : 0) | (j + 1 <= NI ? RP_LOAD1 | RP_STORE1 : 0));
+                it = seen.emplace(std::make_pair(jlo, jhi), close(c, p)).first;
+            }
+            steps.push_back(it->second);
+        }
+        std::vector<FieldDesc> init;
+        for (int pass = 0; pass < 2; pass++)  // right-moving emission; then the left-moving one added
+            for (int f = 0; f < nb; f++)
+                for (int i = 1; i <= NI; i++) {
+                    FieldDesc d{off(f, i), 2 * i + pass, -1, f, 0};
+                    if (pass == 1 && i == NI) d.ktab = 2 * Nd;
+                    if (reflect_h && !emit_h) d.ktab = pass == 1 && i == NI ? 0 : -1;
+                    init.push_back(d);
+                }
+        auto put = [&](DevBuf& d, const void* p, size_t bytes) {
+            if (d.bytes < bytes) d.alloc(bytes);
+            upload(d.p, p, bytes, s);
+        };
+        put(dinit, init.data(), sizeof(FieldDesc) * init.size());
+        put(dlist, cl.data(), sizeof(FieldDesc) * cl.size());
+        put(dpair, pl.data(), sizeof(RdPair) * pl.size());
+        auto go = [&](const Step& t) {
+            rd_cols(sh, red.template col_args<S>(Fp, dlist.as<FieldDesc>() + t.c), t.nc, s);
+            rd_pairs(sh, red.template pair_args<S>(Fp, dpair.as<RdPair>() + t.p, dcoef.as<zd>(), rt), t.np, s);
+        };
+        const int ni = nb * NI;
+        const zd* ap = src ? nullptr : damp.as<zd>();
+        rd_init(sh, red.template init_args<S>(Fp, dinit.as<FieldDesc>(), ap, src, false), ni, s);
+        for (const Step& t : prologue) go(t);
+        rd_init(sh, red.template init_args<S>(Fp, dinit.as<FieldDesc>() + ni, ap, src, true), ni, s);
+        for (const Step& t : steps) go(t);
+        const zd one = cmk<double>(1.0, 0.0);
+        for (int side = 0; side < sides; side++) {
+            const bool right = side == 0;
+            red.propagate_sums(right ? 0 : nb, right ? last : first, sizeof(S) == 4, out.as<zd>());
+            // right: E[Nd-1] right-moving + rl E[Nd-1] left-moving; left: both of E[0]
+            const zd t = right ? tr[Nd - 2] : tl[0], b1 = right ? rl[Nd - 2] : one;
+            const int e = right ? Nd - 1 : 0;
+            const zd *base0 = nullptr, *base1 = nullptr;
+            if (emit_h) {
+                base0 = src + K * (2 * (size_t)e);
+                base1 = src + K * (2 * (size_t)e + 1);
+            } else if (reflect_h && right) {
+                base1 = src + K;
+            }
+            const zd b0 = src ? one : cadd(amp[2 * e], cmul(b1, amp[2 * e + 1]));
+            hipLaunchKernelGGL(k_ch_output, dim3(grid1d(K, 256, 1024), nb), dim3(256), 0, s, out.as<zd>(), K, g.nx, base0,
+                               base1, b0, b1, t, g.X.as<double>(), g.Y.as<double>(), diskR * diskR, src ? 0 : 1);
+            BF_CHECK_LAUNCH();
+            download((right ? out_right : out_left) + 2 * K * f0, out.p, sizeof(zd) * K * nb, s);
+            BF_HIP(hipStreamSynchronize(s));
+        }
+    }
+}
+
 template <typename T>
 void cheerleader_run(bf_ctx* ctx, const bf_setup* st, const bf_coords* co, double amin, int nmax, const double* fr,
                      int nfr, int kind, const double* emit_h, const double* reflect_h, double diskR, double* out_right,
@@ -2404,6 +2635,14 @@ void cheerleader_run(bf_ctx* ctx, const bf_setup* st, const bf_coords* co, doubl
         rr[i] = r[i];
         tl[i] = cmk<double>(1.0 - r[i].re, -r[i].im);
         tr[i] = cmk<double>(1.0 + r[i].re, r[i].im);
+    }
+    if constexpr (!std::is_same<T, f32pure>::value) {
+        RdShape sh;
+        if (Nd >= 4 && Reduced::usable(g, kind, amin, nmax, diskR, sh)) {
+            cheerleader_reduced<T>(ctx, g, sh, st, nmax, fr, nfr, kind, emit_h, reflect_h, diskR, surf.as<zd>(), rl, rr, tl,
+                                   tr, out_right, out_left);
+            return;
+        }
     }
     const size_t per = sizeof(cplx<S>) * K * Nd;
     // Gauss-Seidel is sequential over regions: a launch touches only the one or

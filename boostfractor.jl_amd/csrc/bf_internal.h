@@ -6,7 +6,6 @@
 #include <cstdint>
 #include <cstring>
 #include <map>
-#include <iterator>
 #include <memory>
 #include <mutex>
 #include <stdexcept>
@@ -40,7 +39,7 @@ struct Error : std::runtime_error {
 // ~9 us each (milliseconds for hundreds of MB, and hipFree waits for the device).
 // Everything a context does is ordered on its one stream, so memory that work queued
 // earlier may still use can be handed out again at once.  The pool keeps at most
-// KEEP bytes (the smallest blocks first), frees them all when an allocation fails and
+// KEEP bytes (the last ones given back), frees them all when an allocation fails and
 // when the context is destroyed; blocks that come back later are freed directly.
 // A plan may be destroyed on another thread than its context's calls: the lock.
 class DevPool {
@@ -56,7 +55,7 @@ class DevPool {
         std::lock_guard<std::mutex> lk(mu);
         auto it = blocks.find(block);
         if (it == blocks.end()) return nullptr;
-        void* p = it->second;
+        void* p = it->second.first;
         blocks.erase(it);
         kept -= block;
         return p;
@@ -68,34 +67,37 @@ class DevPool {
             if (closed || block > KEEP) {
                 out.push_back(p);
             } else {
-                blocks.emplace(block, p);
+                blocks.emplace(block, std::make_pair(p, ++turn));
                 kept += block;
-                while (kept > KEEP) {  // the largest go
-                    auto it = std::prev(blocks.end());
-                    out.push_back(it->second);
-                    kept -= it->first;
-                    blocks.erase(it);
+                while (kept > KEEP) {  // the block that lay unused longest goes
+                    auto old = std::min_element(blocks.begin(), blocks.end(), [](const auto& a, const auto& b) {
+                        return a.second.second < b.second.second;
+                    });
+                    out.push_back(old->second.first);
+                    kept -= old->first;
+                    blocks.erase(old);
                 }
             }
         }
         for (void* q : out) (void)hipFree(q);
     }
     void trim(bool close = false) {
-        std::multimap<size_t, void*> out;
+        decltype(blocks) out;
         {
             std::lock_guard<std::mutex> lk(mu);
             out.swap(blocks);
             kept = 0;
             closed = closed || close;
         }
-        for (auto& b : out) (void)hipFree(b.second);
+        for (auto& b : out) (void)hipFree(b.second.first);
     }
     ~DevPool() { trim(true); }
 
   private:
     std::mutex mu;
-    std::multimap<size_t, void*> blocks;
+    std::multimap<size_t, std::pair<void*, uint64_t>> blocks;  // by size: address, turn it came back
     size_t kept = 0;
+    uint64_t turn = 0;
     bool closed = false;
 };
 // pool of the context whose call runs on this thread (null outside a call)
@@ -431,6 +433,7 @@ struct Grid {
     DevBuf axes;         // X, Y, kX, kY, double: one upload
     View X, Y, kX, kY;
     std::vector<double> hX, hY, hkX, hkY;  // host copies
+    void host(const bf_coords* c);  // sizes and host copies only
     void upload(const bf_coords* c, hipStream_t s);
     size_t K() const { return (size_t)nx * ny; }
 };

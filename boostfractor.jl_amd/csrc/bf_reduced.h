@@ -15,6 +15,11 @@
 // the masked fields are summed first (FP64, on the window, transformed along x) and
 // the sum is propagated once on the whole grid.
 //
+// The k range of an even grid is symmetric about half a bin, k = (m + 1/2) dk (about a bin
+// for an odd one), so h(d) = exp(-i pi d / N) g(d) with an even g: fields carried with the
+// factor exp(i pi y / N) (which commutes with masks, surfaces and boundaries) see the even
+// kernel g, whose tables are mirror symmetric and stored as quarters.
+//
 // Lines have M = 16 R points.  Thread t of 16 holds the samples t + 16 m (m < R, of
 // which at most half lie in the window), thread k1 of R the wavenumbers k1 + R k2
 // (k2 < 16): one exchange through LDS per transform, radix R on one side and radix 16
@@ -27,16 +32,31 @@ namespace bf {
 struct RdShape {
     int Ry = 0, Rx = 0;            // radices: lines of 16 Ry (columns) and 16 Rx (rows) points
     int y0 = 0, by = 0, x0 = 0, bx = 0;  // window in the grid
+    double ey = 0, ex = 0;         // phase per sample in units of pi: 1/ny, 1/nx on even grids, else 0
+    bool quarter = false;          // mirror-symmetric k range: quarter tables
     int My() const { return 16 * Ry; }
     int Mx() const { return 16 * Rx; }
     size_t field() const { return (size_t)by * Mx(); }  // elements of a stored field: window rows, wavenumbers along x
-    size_t table() const { return (size_t)My() * Mx(); }
+    size_t points() const { return (size_t)My() * Mx(); }
+    size_t table() const { return quarter ? (size_t)(My() / 2 + 1) * (Mx() / 2 + 1) : points(); }
 };
 // smallest radix whose lines hold the window's convolution, or 0
 inline int rd_radix(int b) {
     for (int R : {4, 5, 6, 8, 10, 12, 16, 20})
         if (2 * b - 1 <= 16 * R) return R;
     return 0;
+}
+
+// Position of wavenumber k = k1 + R q in a stored line: complex64 lines keep the q = 2 j and
+// 2 j + 1 of a k1 side by side, one 16-byte access of the row pass.
+template <bool PAIR>
+__host__ __device__ constexpr int rd_pos(int R, int k1, int q) {
+    return PAIR ? (q >> 1) * 2 * R + 2 * k1 + (q & 1) : k1 + R * q;
+}
+// wavenumber stored at position x
+template <bool PAIR>
+__host__ __device__ constexpr int rd_wavenumber(int R, int x) {
+    return PAIR ? (x % (2 * R) >> 1) + R * (2 * (x / (2 * R)) + (x & 1)) : x;
 }
 
 // column pass entries: FieldDesc.off field, .ktab table, .rtab slot of the running sum (-1: none)
@@ -54,8 +74,9 @@ template <typename S>
 struct RdColArgs {
     cplx<S>* F;
     const FieldDesc* fd;
-    int Mx, by;
-    const zd* tab;  // [table][My][Mx]
+    int Rx, by;
+    const zd* tab;  // [table][My][Mx], or the quarters [table][My/2+1][Mx/2+1]
+    int quarter;
     zd* sum;        // [slot][by][Mx]
     const zd* tw;   // exp(-2 pi i t k1 / My) at [k1][t]
 };
@@ -81,6 +102,7 @@ struct RdInitArgs {
     size_t K;
     const uint32_t* keep;
     const zd* tw;
+    double ex, ey;
     int add;  // add to the stored fields
 };
 // a sum back to the window, written into whole-grid fields [slot][ny][nx]
@@ -90,14 +112,18 @@ struct RdFinalArgs {
     int by, bx, x0, y0, nx;
     size_t K;
     const zd* tw;
+    double ex, ey;
 };
 
 template <typename S> void rd_cols(const RdShape& sh, const RdColArgs<S>& a, int nf, hipStream_t s);
 template <typename S> void rd_pairs(const RdShape& sh, const RdPairArgs<S>& a, int n, hipStream_t s);
 template <typename S> void rd_init(const RdShape& sh, const RdInitArgs<S>& a, int nf, hipStream_t s);
-void rd_final(const RdShape& sh, const RdFinalArgs& a, int n, hipStream_t s);
-// h [ntab][ny][nx] cut to the window's offsets: out [ntab][My][Mx], times 1/(My Mx)
+// pair: the sum is of complex64 fields
+void rd_final(const RdShape& sh, const RdFinalArgs& a, int n, bool pair, hipStream_t s);
+// h [ntab][ny][nx] cut to the window's offsets and made even: out [ntab][My][Mx], times 1/(My Mx)
 void rd_crop(const RdShape& sh, const zd* h, int nx, int ny, int ntab, zd* out, hipStream_t s);
+// the quarters of ntab tables [My][Mx]
+void rd_quarter(const RdShape& sh, const zd* full, int ntab, zd* out, hipStream_t s);
 // twiddles [k1 < R][t < 16]
 void rd_twiddles(int R, zd* out, hipStream_t s);
 

@@ -93,3 +93,31 @@ def test_history_amin_and_short_runs_keep_the_whole_grid():
     assert np.array_equal(a, b)
     a, b = _both(lambda: B.dancer(0, 3, sb, c, f=20e9, diskR=DISKR))
     assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("nx,ny,shift", [(128, 128, 0), (101, 101, 0), (256, 128, 30), (150, 100, 0)])
+@pytest.mark.parametrize("prec", ["fp64", "mixed"])
+@pytest.mark.parametrize("ndisk", [1, 3])
+def test_cheerleader_on_the_window(nx, ny, shift, prec, ndisk):
+    c = _grid(nx, ny, shift)
+    sb = W.rough_booster(c, ndisk=ndisk, seed=21)
+    refl = np.exp(-(c.X[None] ** 2 + c.Y[:, None] ** 2) / 0.1 ** 2) * np.exp(3j * c.X[None])
+    rng = np.random.default_rng(4)
+    emit = rng.standard_normal((len(sb.distance), 2, ny, nx)) + 1j * rng.standard_normal((len(sb.distance), 2, ny, nx))
+    sb.r[0] = 0.7 + 0.1j  # so that something leaves on the left
+    for kw in ({}, {"reflect": refl}, {"emit": emit}):
+        a, b = _both(lambda: B.cheerleader(0, 9, sb, c, f=[19.9e9, 20e9, 20.3e9], diskR=DISKR, precision=prec,
+                                           returnboth=True, **kw))
+        for x, y in zip(a, b):
+            assert np.any(y != 0) and rel(x, y) < TOL[prec]
+    a, b = _both(lambda: B.cheerleader(0, 9, sb, c, f=20e9, prop=B.propagatorNoTilts, diskR=DISKR, precision=prec))
+    assert rel(a, b) < TOL[prec]
+
+
+def test_cheerleader_amin_and_short_runs_keep_the_whole_grid():
+    c = _grid(128, 128)
+    sb = _booster(c, False, 22)
+    a, b = _both(lambda: B.cheerleader(0.05, 30, sb, c, f=20e9, diskR=DISKR))
+    assert np.array_equal(a, b)
+    a, b = _both(lambda: B.cheerleader(0, 2, sb, c, f=20e9, diskR=DISKR))
+    assert np.array_equal(a, b)
