@@ -33,6 +33,14 @@ struct ModesDev {
 struct ModeCache {
     DevBuf G, Fhat, FhatM;
     bool haveG = false, haveF = false;
+    // Support of the patterns: the Ks grid points where some pattern is not zero (Bessel modes: the aperture,
+    // 7% of a 1 m grid).  `compact`: the patterns at those points only, patc[n][C Ks], for Gram sums.
+    bool haveSup = false, compact = false;
+    bool maskedSame = false;  // all of them inside the aperture: masked patterns = patterns, FhatM is not formed
+    size_t Ks = 0;
+    std::vector<int> hsup;
+    DevBuf sup, supw, patc;  // points; bit p of word p / 64; patterns
+    const DevBuf& masked() const { return maskedSame ? Fhat : FhatM; }
     DevBuf Ginv;  // inv(G), formed by the first flat-disk flush that needs it
     bool haveGinv = false, ginv_ok = false;
     // Parseval regions by k-bin group: bins with equal (kx^2, ky^2) (and, on a
@@ -54,7 +62,7 @@ struct ModeCache {
     DevBuf goff, gbin;  // group g holds bins gbin[goff[g] .. goff[g+1])
     // forget everything computed from the patterns (keeps the grouping)
     void reset_data() {
-        haveG = haveF = haveH = haveGinv = false;
+        haveG = haveF = haveH = haveGinv = haveSup = false;
         reset_series();
     }
     // coefficient matrices of the spacing series (parseval_flush) formed so far in this run, by
