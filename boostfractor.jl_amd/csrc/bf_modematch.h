@@ -58,6 +58,7 @@ struct ModeCache {
     int ngroups = 0;
     DevBuf gkx, gky;    // representative kX, kY of each group (double)
     double gk2max = 0.0;  // max over groups of kX^2 + kY^2
+    std::vector<double> gk2;  // kX^2 + kY^2 of the groups, ascending
     int gmax = 0;         // most bins in one group
     DevBuf goff, gbin;  // group g holds bins gbin[goff[g] .. goff[g+1])
     // forget everything computed from the patterns (keeps the grouping)

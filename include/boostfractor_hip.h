@@ -113,7 +113,8 @@ int bf_ctx_kernel_time(bf_ctx *ctx, const char *kernel, double *ms, int64_t *lau
  * transforms, wavefront order), "graph" (dancer plans replay HIP graphs),
  * "parseval_groups", "disk_expansion", "parseval_series" (transformer work
  * reductions: k-bin groups, disks from the Gram matrix, air gaps by a series
- * in the spacing), "series_inverse" (the gaps' inverses by the inverse's
+ * in the spacing), "parseval_nodes" (with parseval_series: air gaps and series
+ * coefficients of a band of frequencies interpolated in k0^2), "series_inverse" (the gaps' inverses by the inverse's
  * series in flat sweep chunks; a run whose series fails its convergence check
  * is redone with LU inverses, which 2 forces), "chain_tile" (register-tiled
  * chain kernels for n = 9, 15, 25, 45), "chain_mfma" (chain on the matrix

@@ -1,0 +1,48 @@
+"""Parseval products over a band of frequencies, interpolated in k0^2 at
+Chebyshev nodes (option parseval_nodes), against the direct products and the
+CPU oracle.  Narrow and wide bands, gaps of 0 to 0.4 m (waves that propagate
+grow on the interpolation's ellipse with the gap), grids with few and many
+k-bin groups, frequencies in any order and repeated, and gaps the
+interpolation has to leave alone: a lossy one and, with the propagator that
+keeps it, a permittivity with imaginary part +0.
+"""
+import numpy as np
+import pytest
+
+import BoostFractor as B
+from BoostFractor import workloads as W
+from helpers import DISKR, O, ocoords, rel
+from test_gpu_support import _modes
+
+pytestmark = pytest.mark.gpu
+
+
+def _stack(n, eps):
+    """gaps of several lengths, one of them with its own permittivity"""
+    coords = W.grid_coords(n)
+    dist = np.array([0.0, 8e-3, 1e-3, 0.0, 1e-3, 2.5e-2, 1e-3, 0.4, 1e-3, 7.9e-3])
+    e = np.array([np.nan, 1, 24, 1, 24, 1, 24, 1, 24, eps], dtype=complex)
+    return coords, B.SeedSetupBoundaries(coords, diskno=4, distance=dist, epsilon=e)
+
+
+@pytest.mark.parametrize("lo,hi,nf", [(19.99e9, 20.01e9, 40), (19.5e9, 20.5e9, 100), (12e9, 24e9, 64), (20e9, 20.2e9, 9)])
+@pytest.mark.parametrize("n", [33, 128])
+@pytest.mark.parametrize("kind", [(B.propagator, O.PROP_PROPAGATOR), (B.propagatorNoTilts, O.PROP_NOTILTS)],
+                         ids=["propagator", "notilts"])
+def test_interpolated_products(engine_options, n, lo, hi, nf, kind):
+    coords, sb = _stack(n, complex(1.0, -1e-3))
+    modes = _modes(coords, DISKR)
+    freqs = np.random.default_rng(nf).permutation(np.append(np.linspace(lo, hi, nf - 1), lo))
+    gaps = [1, 3, 5, 7, 9]
+    got = B.calc_propagation_matrices(sb, coords, modes, f=freqs, prop=kind[0], diskR=DISKR)
+    engine_options(parseval_nodes=0)
+    want = B.calc_propagation_matrices(sb, coords, modes, f=freqs, prop=kind[0], diskR=DISKR)
+    for q in range(nf):
+        for r in gaps:
+            assert rel(got[q][r], want[q][r]) < 1e-13, (q, r, rel(got[q][r], want[q][r]))
+    pat, kt = modes.patterns_flat()[:, 0], modes.mode_kt.reshape(-1)
+    for q in (0, nf // 2):
+        for r in gaps:
+            o = O.propagation_matrix(sb.distance[r], DISKR, sb.eps[r], 0.0, 0.0, np.zeros((n, n), dtype=complex),
+                                     B.wavelength(freqs[q]), ocoords(coords), pat, kt, kind[1])
+            assert rel(got[q][r], o) < 1e-10, (q, r)
