@@ -1329,7 +1329,7 @@ struct Reduced {
 
     // The window of the grid's aperture, when the reduced convolution is at most 3/4 of the grid (a power
     // of two) or no larger than it (other sizes, whose own lines take 2 n^2 flop on the matrix cores).
-    // Measured at 0.39 of 256^2 and 512^2 (1.5 and 2.2 times faster) and 0.63 of 101^2 (2.5 times); 192 of
+    // Measured at 0.39 of 256^2 and 512^2 (1.5 and 2.2 times faster) and 0.40 of 101^2 (2.5 times); 192 of
     // 256 points a line, 0.56, is the next larger shape below the grid's own.
     static bool shape(const Grid& g, double diskR, RdShape& sh) {
         int lo, hi;

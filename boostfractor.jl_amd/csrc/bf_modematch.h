@@ -183,6 +183,9 @@ std::vector<zd> eps_fixed(const bf_setup* st);
 // chain steps of one geometry at one frequency (regions Nreg-1 .. 1, :311-341)
 void append_chain_steps(const std::vector<zd>& eps, int nreg, std::vector<ChainStep>& steps);
 
+// inv(P) of the matrices `sel`
+void inverses(bf_ctx* ctx, int n, const zd* P, zd* Pinv, const std::vector<int>& sel, Stager* st = nullptr);
+
 // inv(P) of the matrices `sel`, then one chain per job; boost (and refl) [njobs][n]
 void inverse_and_chains(bf_ctx* ctx, int n, zd* P, zd* Pinv, const std::vector<int>& sel,
                         const std::vector<ChainJob>& jobs, const std::vector<ChainStep>& steps, const zd* e0,

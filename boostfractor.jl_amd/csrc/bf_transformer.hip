@@ -3977,18 +3977,21 @@ void append_chain_steps(const std::vector<zd>& eps, int nreg, std::vector<ChainS
     for (int q = 0; q < nreg - 1; q++) steps.push_back(chain_step(eps.data(), nreg, q));
 }
 
+void inverses(bf_ctx* ctx, int n, const zd* P, zd* Pinv, const std::vector<int>& sel, Stager* st) {
+    if (sel.empty()) return;
+    DevBuf& dsel = scratch_buf(ctx, SB_SEL, sizeof(int) * sel.size());
+    stage_upload(st, dsel.p, sel.data(), sizeof(int) * sel.size(), ctx->stream);
+    TimedLaunch tl(ctx, "inverse", (8.0 / 3.0 + 8.0) * (double)n * n * n * (double)sel.size());
+    launch_inverse(ctx, P, Pinv, n, dsel.as<int>(), sel.size());
+}
+
 void inverse_and_chains(bf_ctx* ctx, int n, zd* P, zd* Pinv, const std::vector<int>& sel,
                         const std::vector<ChainJob>& jobs, const std::vector<ChainStep>& steps, const zd* e0,
                         const zd* reflect, zd* boost, zd* refl, Stager* st, const ChainSrc* disks) {
     hipStream_t s = ctx->stream;
     const size_t nn = (size_t)n * n;
     const int N2 = 2 * n;
-    DevBuf& dsel = scratch_buf(ctx, SB_SEL, sizeof(int) * sel.size());
-    stage_upload(st, dsel.p, sel.data(), sizeof(int) * sel.size(), s);
-    if (!sel.empty()) {
-        TimedLaunch tl(ctx, "inverse", (8.0 / 3.0 + 8.0) * (double)n * n * n * (double)sel.size());
-        launch_inverse(ctx, P, Pinv, n, dsel.as<int>(), sel.size());
-    }
+    inverses(ctx, n, P, Pinv, sel, st);
     const size_t nj = jobs.size();
     const bool lds = n <= CHAIN_LDS_MAX;
     // Blocks start roughly in index order, so a batch of chains of unequal length (geometries with

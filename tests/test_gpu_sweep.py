@@ -138,3 +138,20 @@ def test_boostfactor_cost_matches_oracle_composition():
         assert abs(costs[c] / want - 1) < 1e-9, (c, costs[c], want)
         one = B.calc_boostfactor_cost(d, itp, freqs, sb.copy(), coords, modes, m_reflect, diskR=DISKR)
         assert one == pytest.approx(costs[c], rel=1e-14)
+
+
+@pytest.mark.parametrize("chunk_bytes", [None, 20000])
+def test_spacing_candidates_together_and_alone(engine_options, chunk_bytes):
+    """candidates share the inverses of regions at the first one's spline point (every disk, the last gap, a gap
+    that was not moved): bit for bit the results of one call per candidate"""
+    if chunk_bytes:
+        engine_options(batch_bytes=chunk_bytes)
+    coords, sb, modes = _setup(ndisk=2)
+    spacing = np.linspace(-2e-4, 2e-4, 5)
+    itp = B.construct_prop_matrix_interpolation(_grid(coords, sb, modes, spacing, [19.9e9, 20.1e9]), spacing)
+    emit = B.axion_induced_modes(coords, modes, diskR=DISKR)
+    eps = np.where(np.isnan(sb.eps), 1e30, sb.eps)
+    cands = np.array([[1e-4, -0.5e-4], [1e-4, 0.3e-4], [0.0, -0.5e-4], [1e-4, -0.5e-4], [-1.1e-4, 0.7e-4]])
+    both = itp.transformer(cands, eps, emit)
+    for c in range(len(cands)):
+        assert np.array_equal(both[c], itp.transformer(cands[c:c + 1], eps, emit)[0]), c
