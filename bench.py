@@ -11,8 +11,9 @@ split the geometries into K disjoint contiguous slices, so K steps cover the
 whole sweep once; `value` is the whole sweep's points over the timed time.
 The sweep has no reduced-precision path (its products run on FP64 MFMA), so
 `mixed_over_fp64` is 1.0.  The dancer workloads (`--workload dancer`,
-`dancer512`) time a complex64-storage path against FP64 and report the ratio
-and the beta^2 error of every point.
+`dancer512`) time the mixed path against FP64 and report the ratio and the
+beta^2 error of every point (bounces on the aperture's window keep complex128
+fields in both).
 
 Kernel timing: the timed steps run without instrumentation; one more step
 then records HIP events on the engine's stream around every launch of the
@@ -20,9 +21,9 @@ kernel classes, which gives the kernels' mean launch times.
 
 Roofline: the dominant kernel's executed work per launch over its mean launch
 time (sweep and transformer: FP64 MFMA flops of the grouped-Parseval
-product; dancer: the bounce's algorithmic bytes, every field read once and
-written once per bounce and frequency, 2 F K B_c with F = 82 fields, over
-the two bounce kernels' combined time per frequency-bounce).  `traffic` is
+product; dancer: the bytes of the F = 82 fields on the aperture's window,
+read once and written once by each of the bounce's two passes, over their
+combined time per frequency-bounce).  `traffic` is
 HBM bytes per launch from rocprofv3 FETCH_SIZE / WRITE_SIZE, each scaled by
 the same counter's reading for a copy kernel of known size.
 
@@ -742,20 +743,17 @@ def main():
                                           "p90": float(np.percentile(errf, 90))},
                 "note": "complex64 fields with FP32 FFT, phase and update arithmetic (phase argument in FP64)"}
 
-    # roofline of the mixed path's bounce: a frequency batch's bounce is two launches (column pass, fused
-    # row pass) that together read and write every field once; the bounce's algorithmic bytes are divided
-    # by the two launches' combined mean time (each pass alone moves the same fields, so neither gets the
-    # whole bounce's bytes on its own time)
+    # roofline of the bounce: a frequency batch's bounce is two launches (columns, boundary pairs), each of
+    # which reads and writes every field on the aperture's window once: by rows of Mx wavenumbers, complex128
     col_ms, launches = kt32["col_pass"]
     row_ms, row_launches = kt32["row_pass"]
     avg_ms = (col_ms + row_ms) / launches  # one column + one row launch per frequency batch and bounce
     nb_per_launch = NFREQ * (nmax + 1) / launches  # frequency-bounces per launch pair (one instrumented run)
-    alg_bytes = nb_per_launch * 2 * F * K * 8  # every field read once and written once, complex64
+    by = info32["band"][1] - info32["band"][0]
+    mx = min(16 * r for r in (4, 5, 6, 8, 10, 12, 16, 20) if 16 * r >= 2 * by - 1)
+    fb_bytes = 2 * 2 * F * by * mx * 16
+    alg_bytes = nb_per_launch * fb_bytes
     achieved = alg_bytes / (avg_ms * 1e-3) / 1e9
-    # HBM bytes of both passes per launch pair, from the committed counter summary (256 x 256 only)
-    tc = traffic_from_profile("k_cols_reg", fb32) if N == 256 else None
-    tr = traffic_from_profile("k_dancer_rows_reg4", fb32) if N == 256 else None
-    traffic = (tc + tr) if (tc is not None and tr is not None) else None
     bw_ms = ctx.stream_copy_probe(1 << 30, reps=10)
     stream_gbs = 2 * (1 << 30) / (bw_ms * 1e-3) / 1e9
 
@@ -771,7 +769,7 @@ def main():
         "scaling": "weak",
         "vs_baseline": None,
         "dtype": "f64",
-        "storage": "complex64 fields in HBM (mixed precision: every FFT, phase and boundary update in f64)",
+        "storage": "complex128 fields on the aperture's window (every FFT, phase and boundary update in f64)",
         "data": "synthetic (seeded SplitMix64 booster geometry, axion source from dance_intro)",
         "config": {"workload": f"dancer, 20-disk booster eps=24, {N}x{N} grid over 1 m, {NFREQ} freqs "
                                f"19.5-20.5 GHz, nmax={nmax}, FFT propagator, one batched device-resident sweep",
@@ -779,21 +777,20 @@ def main():
         "fp64": fp64,
         "roofline": {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(achieved / HBM_PEAK_GBS, 4),
-                     "traffic": traffic if traffic is None else int(traffic),
-                     "kernel": "dancer bounce: k_cols_reg (column FFT, exp(-i kz dz)/K, column IFFT) + "
-                               "k_dancer_rows_reg (row IFFT, tilt/surface, boundary update, mask, row FFT)",
+                     "traffic": None,
+                     "kernel": "dancer bounce: k_rd_cols (column FFT, kernel table, column IFFT) + "
+                               "k_rd_pairs (row IFFT, tilt/surface, boundary update, mask, row FFT)",
                      "avg_launch_ms": round(avg_ms, 4),
                      "col_pass_ms": round(col_ms / launches, 4), "row_pass_ms": round(row_ms / row_launches, 4),
                      "alg_bytes_per_launch": int(alg_bytes),
                      # the same algorithmic bytes over the whole step (both bounce kernels, the gaps between
                      # launches and the per-batch setup): the rate a user of the sweep sees
-                     "whole_step_GBs": round(NFREQ * (nmax + 1) * 2 * F * K * 8 / (dt32 / args.steps) / 1e9, 1),
+                     "whole_step_GBs": round(NFREQ * (nmax + 1) * fb_bytes / (dt32 / args.steps) / 1e9, 1),
                      "measured_stream_copy_GBs": round(stream_gbs, 1)},
-        "work_reductions": {"row_band": list(info32["band"]), "rows": N,
-                            "note": "rows outside the aperture band skipped by both passes (exit field kept whole); "
-                                    "band-pruned register FFTs (zero elements and unstored outputs skipped); "
-                                    "identical k-space tables shared, quarter tables for complex64 fields; "
-                                    "not folded into roofline.achieved"},
+        "work_reductions": {"window": [by, mx], "rows": N,
+                            "note": "bounces as circular convolutions on the window that holds the aperture; "
+                                    "identical k-space tables shared, stored as quarters; exit fields summed and "
+                                    "propagated once"},
         "kernel_ms": {k: [round(v[0], 3), v[1]] for k, v in kt32.items()},
     }
     tuned, tune_ms = ctx.tuning_report()
