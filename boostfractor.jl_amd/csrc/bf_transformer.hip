@@ -652,6 +652,93 @@ __global__ void __launch_bounds__(64) k_batched_inverse_wave(const zd* __restric
     wave_each2d(lane, n, n, [&](int j, int i) { dst[i + n * j] = M[i + n * sig[j]]; });
 }
 
+// The same inverse, bit for bit, by four waves for 32 < n <= 48.  LDS holds four to five such matrices on a CU,
+// one wave each with the kernel above: too few to cover the latency of n dependent pivots.  A lane
+// owns a row and the waves share the columns.  4100 matrices of 45 x 45: 1.29 -> 0.62 ms.  At n <= 32 a
+// CU holds ten and more matrices, and half of the lanes would have no row.
+__global__ void __launch_bounds__(256) k_batched_inverse_block(const zd* __restrict__ P, zd* Pinv, int n,
+                                                               const int* __restrict__ sel,
+                                                               const InvSel* __restrict__ bs) {
+    extern __shared__ unsigned char smem_raw[];
+    zd* M = reinterpret_cast<zd*>(smem_raw);  // column-major n x n
+    __shared__ zd colk[INV_WAVE_MAX];
+    __shared__ int piv[INV_WAVE_MAX], sig[INV_WAVE_MAX];
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    const int64_t b = bs ? bs[blockIdx.x].base + (int64_t)blockIdx.y * bs[blockIdx.x].stride
+                         : (sel ? sel[blockIdx.x] : blockIdx.x);
+    const int nn = n * n;
+    const zd* src = P + (size_t)b * nn;
+    for (int e = t; e < nn; e += 256) M[e] = src[e];
+    __syncthreads();
+    for (int k = 0; k < n; k++) {
+        // every wave finds the pivot; wave 0 keeps column k as the swap of rows k and p leaves it
+        double best = -1.0;
+        int bi = k;
+        zd v = cmk<double>(0.0, 0.0);
+        if (lane < n) v = M[lane + n * k];
+        if (lane >= k && lane < n) {
+            const double a = fabs(v.re) + fabs(v.im);
+            if (a > best) { best = a; bi = lane; }
+        }
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) {
+            const double ob = __shfl_xor(best, o);
+            const int oi = __shfl_xor(bi, o);
+            if (ob > best || (ob == best && oi < bi)) { best = ob; bi = oi; }
+        }
+        const int p = bi;
+        const zd d = M[p + n * k];
+        const double den = d.re * d.re + d.im * d.im;
+        const zd r = cmk<double>(d.re / den, -d.im / den);
+        if (t < n) colk[t == k ? p : t == p ? k : t] = v;
+        if (t == 0) piv[k] = p;
+        __syncthreads();
+        // rows k and p swapped, row k scaled by r (its pivot entry becomes r)
+        if (t < n) {
+            const zd u = M[p + n * t];
+            if (p != k) M[p + n * t] = M[k + n * t];
+            M[k + n * t] = t == k ? r : cmul(u, r);
+        }
+        __syncthreads();
+        // row i != k: M[i][j] -= M_old[i][k] M[k][j] (j != k), M[i][k] = -M_old[i][k] r
+        if (lane < n && lane != k) {
+            const zd f = colk[lane];
+            for (int j = wave; j < n; j += 4) {
+                zd* m = M + lane + n * j;
+                *m = j == k ? csub(cmk<double>(0.0, 0.0), cmul(f, r)) : csub(*m, cmul(f, M[k + n * j]));
+            }
+        }
+        __syncthreads();
+    }
+    // undo the row swaps on the columns, in reverse order: result column j is column sig[j]
+    if (t == 0) {
+        for (int j = 0; j < n; j++) sig[j] = j;
+        for (int k = n - 1; k >= 0; k--) {
+            const int q = sig[k];
+            sig[k] = sig[piv[k]];
+            sig[piv[k]] = q;
+        }
+    }
+    __syncthreads();
+    zd* dst = Pinv + (size_t)b * nn;
+    if (lane < n)
+        for (int j = wave; j < n; j += 4) dst[lane + n * j] = M[lane + n * sig[j]];
+}
+
+// inverses of matrices of n <= INV_WAVE_MAX by the kernel for their size; grid and selection as the kernels'
+static void launch_small_inverse(dim3 grid, hipStream_t s, const zd* P, zd* Pinv, int n, const int* sel,
+                                 const InvSel* bs) {
+    const size_t smem = sizeof(zd) * (size_t)n * n;
+    if (n > 32) {
+        allow_lds((const void*)k_batched_inverse_block, smem);
+        hipLaunchKernelGGL(k_batched_inverse_block, grid, dim3(256), smem, s, P, Pinv, n, sel, bs);
+    } else {
+        allow_lds((const void*)k_batched_inverse_wave, smem);
+        hipLaunchKernelGGL(k_batched_inverse_wave, grid, dim3(64), smem, s, P, Pinv, n, sel, bs);
+    }
+    BF_CHECK_LAUNCH();
+}
+
 // ---------------------------------------------------------------------------
 // transfer-matrix chain, one block per job (src/boost_fractor_transformer.jl:326-357)
 // ---------------------------------------------------------------------------
@@ -2120,11 +2207,7 @@ static void launch_inverse(bf_ctx* ctx, const zd* P, zd* Pinv, int n, const int*
     hipStream_t s = ctx->stream;
     if (count == 0) return;
     if (n <= INV_WAVE_MAX) {
-        const size_t smem = sizeof(zd) * (size_t)n * n;
-        allow_lds((const void*)k_batched_inverse_wave, smem);
-        hipLaunchKernelGGL(k_batched_inverse_wave, dim3((unsigned)count), dim3(64), smem, s, P, Pinv, n, dsel,
-                           (const InvSel*)nullptr);
-        BF_CHECK_LAUNCH();
+        launch_small_inverse(dim3((unsigned)count), s, P, Pinv, n, dsel, nullptr);
     } else {
         DevBuf work(sizeof(zd) * (size_t)n * n * count);
         hipLaunchKernelGGL(k_batched_inverse, dim3((unsigned)count), dim3(256), 0, s, P, Pinv, n, work.as<zd>(), dsel);
@@ -3564,11 +3647,7 @@ static void series_form(bf_ctx* ctx, ModeCache& mc, int n, double scale, const s
         stage_upload(st, dsel.p, rows0.data(), sizeof(int) * rows0.size(), s);
         stage_upload(st, dj.p, ij.data(), sizeof(SeriesInvJob) * ij.size(), s);
         TimedLaunch tl(ctx, "sinverse", 8.0 * (double)nn * n * (double)fresh.size() * (1.0 + qmax * (qmax + 1) / 2));
-        const size_t smem1 = sizeof(zd) * nn;
-        allow_lds((const void*)k_batched_inverse_wave, smem1);
-        hipLaunchKernelGGL(k_batched_inverse_wave, dim3((unsigned)fresh.size()), dim3(64), smem1, s, blk, inv, n,
-                           dsel.as<int>(), (const InvSel*)nullptr);
-        BF_CHECK_LAUNCH();
+        launch_small_inverse(dim3((unsigned)fresh.size()), s, blk, inv, n, dsel.as<int>(), nullptr);
         if (n > 8 && n <= 32 && opts().sinv_mfma) {
             const dim3 grid((unsigned)fresh.size(), (unsigned)((n + 15) / 16));
             switch ((n + 3) / 4) {
@@ -4630,14 +4709,9 @@ static void flat_launch(bf_ctx* ctx, bf_transformer_batch_plan* pl, int set, Mod
         DevBuf& di = scratch_buf(ctx, SB_FINV, sizeof(InvSel) * bs.size());
         stage_upload(st, di.p, bs.data(), sizeof(InvSel) * bs.size(), s);
         TimedLaunch tl(ctx, "inverse", (8.0 / 3.0 + 8.0) * (double)n * n * n * (double)bs.size() * nf);
-        const size_t smem = sizeof(zd) * nn;
-        allow_lds((const void*)k_batched_inverse_wave, smem);
-        for (size_t i0 = 0; i0 < bs.size(); i0 += 65535) {
-            const size_t ni = std::min<size_t>(65535, bs.size() - i0);
-            hipLaunchKernelGGL(k_batched_inverse_wave, dim3((unsigned)ni, (unsigned)nf), dim3(64), smem, s, P, Pinv,
-                               n, (const int*)nullptr, di.as<InvSel>() + i0);
-            BF_CHECK_LAUNCH();
-        }
+        for (size_t i0 = 0; i0 < bs.size(); i0 += 65535)
+            launch_small_inverse(dim3((unsigned)std::min<size_t>(65535, bs.size() - i0), (unsigned)nf), s, P, Pinv, n,
+                                 nullptr, di.as<InvSel>() + i0);
     }
     inverse_and_chains(ctx, n, P, Pinv, std::vector<int>(), fw.jobs, fw.steps, pl->de0[set].as<zd>(), nullptr, dboost,
                        nullptr, st, disk_src.ph ? &disk_src : nullptr);
