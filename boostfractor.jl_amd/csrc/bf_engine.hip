@@ -1548,6 +1548,12 @@ static bool quarter_tables_ok(const bf_coords* co, int kind) {
            (n & (n - 1)) == 0 && k_mirrored(co->kX, co->nx) && k_mirrored(co->kY, co->ny);
 }
 
+// Whether a dancer with FP64 arithmetic runs its bounces on the aperture's window (sh: its shape)
+static bool dancer_window(const Grid& g, int nreg, double amin, int nmax, int kind, double diskR,
+                          const DancerOptions& o, RdShape& sh) {
+    return o.window && (o.immediatesum || nmax == 0) && nreg > 2 && Reduced::usable(g, kind, amin, nmax, diskR, sh);
+}
+
 template <typename T>
 struct DancerPlan : DancerPlanBase {
     BF_TYPES(T);
@@ -1664,8 +1670,8 @@ struct DancerPlan : DancerPlanBase {
             aperture_range(g.hY, g.hX, diskR, band_lo, band_hi);
         nslices = opt.immediatesum ? 1 : nmax + 1;
         RdShape rsh;
-        const bool rd = std::is_same<T, double>::value && nslices == 1 && R >= 2 &&
-                        Reduced::usable(g, kind, amin, nmax, diskR, rsh);
+        const bool rd =
+            std::is_same<T, double>::value && dancer_window(g, st->nreg, amin, nmax, kind, diskR, opt, rsh);
         const bool qtab = !rd && quarter_tables_ok<T>(co, kind);
         // Frequency batch: what one bounce of a batch touches (the band rows of every
         // field, plus one k-space table per distinct (eps, dz)) is kept near
@@ -2102,11 +2108,11 @@ static DancerPlanBase* make_dancer_plan_fixed(bf_ctx* ctx, const bf_setup* st, c
     // On the window mixed precision keeps complex128 fields too: complex64 ones are 12% faster (the 20-disk
     // booster, 256^2, 20 frequencies: 46.7 against 53.1 ms; 512^2, 4: 21.2 against 23.8) but round the
     // emitted fields 0.7 to 1.35 times as far as the whole grid's mixed passes and their power up to twice.
-    if (precision == BF_PREC_MIXED && st->nreg > 2 && (o.immediatesum || nmax == 0)) {
+    if (precision == BF_PREC_MIXED) {
         Grid g;
         g.host(co);
         RdShape sh;
-        if (Reduced::usable(g, kind, amin, nmax, diskR, sh)) precision = BF_PREC_FP64;
+        if (dancer_window(g, st->nreg, amin, nmax, kind, diskR, o, sh)) precision = BF_PREC_FP64;
     }
     if (precision == BF_PREC_MIXED) {
         auto* p = new DancerPlan<float>();
@@ -2127,19 +2133,25 @@ static DancerPlanBase* make_dancer_plan_fixed(bf_ctx* ctx, const bf_setup* st, c
 // FFTW.fft! calls, src/boost_fractor.jl:163-164, plan by estimate): short runs of the plan's own inputs
 // (nmax cut to TUNE_NMAX, the frequencies cut to a few batches) time candidate
 // frequency batches around the cache-size heuristic, then column-pass tiles,
-// then row-pass rows per block (coordinate descent), per shape key.
+// then row-pass rows per block (coordinate descent), per shape key.  The key names
+// the path: a batch of window fields is far too large a batch of whole-grid ones.
+// Where the solver has both paths the whole grid's key carries a mark of its own, so
+// that no entry is read that was stored without one, from either path.
 static std::string dancer_tune_key(const bf_coords* co, const bf_setup* st, int precision, int kind, double amin,
-                                   int nfr, const DancerOptions& o) {
+                                   int nfr, const DancerOptions& o, bool window, const RdShape& sh) {
+    const bool both = precision != BF_PREC_FP32 && amin == 0.0 && st->nreg > 2 &&
+                      (kind == BF_PROP_PROPAGATOR || kind == BF_PROP_NOTILTS);
     return "dancer p" + std::to_string(precision) + " " + std::to_string(co->nx) + "x" + std::to_string(co->ny) +
            " reg" + std::to_string(st->nreg) + " k" + std::to_string(kind) + " a" + std::to_string(amin != 0.0) +
            " f" + std::to_string(std::min(nfr, 64)) + " s" + std::to_string(o.returnsum) +
            std::to_string(o.immediatesum) + " e" + std::to_string(o.emit != nullptr) +
-           std::to_string(o.reflect != nullptr);
+           std::to_string(o.reflect != nullptr) +
+           (window ? " w" + std::to_string(sh.bx) + "x" + std::to_string(sh.by) : both ? " g" : "");
 }
 
 static void tune_dancer(bf_ctx* ctx, const bf_setup* st, const bf_coords* co, double amin, int nmax,
                         const double* fr, int nfr, int kind, double diskR, int precision, const DancerOptions& o,
-                        const std::string& key) {
+                        bool window, const std::string& key) {
     constexpr int TUNE_NMAX = 20;
     const auto t_start = std::chrono::steady_clock::now();
     hipStream_t s = ctx->stream;
@@ -2147,6 +2159,7 @@ static void tune_dancer(bf_ctx* ctx, const bf_setup* st, const bf_coords* co, do
     base.graph = 0;
     base.returnsum = 1;
     base.immediatesum = 1;
+    base.window = window ? 1 : 0;  // (a summed run of a history plan stays on the whole grid)
     const int nm = std::min(nmax, TUNE_NMAX);
     // the heuristic batch, from a plan that picks it itself
     int fb0;
@@ -2177,6 +2190,16 @@ static void tune_dancer(bf_ctx* ctx, const bf_setup* st, const bf_coords* co, do
         const double tt = time_of(t);
         if (tt < tbest) { tbest = tt; best = t; }
     }
+    auto store = [&] {
+        ctx->tuned[key] = {best.freq_batch, best.col_tx, best.rows};
+        ctx->tune_ms +=
+            std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t_start).count();
+        save_tuned(ctx, key);
+    };
+    if (window) {  // its passes have no other shapes
+        store();
+        return;
+    }
     // column tile (columns per column-pass block; the kernel's default is 128 bytes of a line) and rows
     // per row-pass block (default 128 threads): halved and doubled, in the kernels' valid ranges
     const int esize = precision == BF_PREC_FP64 ? 16 : 8;
@@ -2196,17 +2219,21 @@ static void tune_dancer(bf_ctx* ctx, const bf_setup* st, const bf_coords* co, do
         const double tt = time_of(t);
         if (tt < tbest) { tbest = tt; best = t; }
     }
-    ctx->tuned[key] = {best.freq_batch, best.col_tx, best.rows};
-    ctx->tune_ms += std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t_start).count();
-    save_tuned(ctx, key);
+    store();
 }
 
 DancerPlanBase* make_dancer_plan(bf_ctx* ctx, const bf_setup* st, const bf_coords* co, double amin, int nmax,
                                  const double* fr, int nfr, int kind, double diskR, int precision,
                                  const DancerOptions& o) {
     if (opts().autotune && o.freq_batch == 0 && o.col_tx == 0 && o.rows == 0 && nmax >= 1) {
-        const std::string key = dancer_tune_key(co, st, precision, kind, amin, nfr, o);
-        if (!ctx->tuned.count(key)) tune_dancer(ctx, st, co, amin, nmax, fr, nfr, kind, diskR, precision, o, key);
+        Grid g;
+        g.host(co);
+        RdShape sh;
+        const bool window =
+            precision != BF_PREC_FP32 && dancer_window(g, st->nreg, amin, nmax, kind, diskR, o, sh);
+        const std::string key = dancer_tune_key(co, st, precision, kind, amin, nfr, o, window, sh);
+        if (!ctx->tuned.count(key))
+            tune_dancer(ctx, st, co, amin, nmax, fr, nfr, kind, diskR, precision, o, window, key);
         const std::vector<int64_t>& v = ctx->tuned[key];
         if (v.size() == 3) {
             DancerOptions t = o;

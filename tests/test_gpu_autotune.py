@@ -3,6 +3,7 @@ result beyond rounding, a plan built with the picked shapes set explicitly is
 identical bit for bit, and a tuning file written by one context is read by the
 next, which then times nothing."""
 import math
+from concurrent.futures import ThreadPoolExecutor
 
 import numpy as np
 import pytest
@@ -68,6 +69,41 @@ def test_dancer_autotune_shapes(tmp_path, prec, tol):
             ctx2.close()
     finally:
         ctx.close()
+
+
+def test_dancer_autotune_per_path():
+    """Each path is tuned for itself: short runs, history plans and reduced=0 run on the whole grid, 8 and
+    more summed bounces on the aperture's window, whose shape follows diskR and whose passes have no tiles
+    to choose.  A line of a tuning file that names no path is read by neither."""
+    coords = W.grid_coords(128)
+    sb = W.booster(coords, ndisk=2, seed=1702)
+    freqs = [19.9e9, 20.0e9, 20.1e9]
+
+    def run():
+        ctx = B.context()  # of this thread: nothing tuned yet
+
+        def key(nmax, diskR=DISKR, **kw):
+            before = set(ctx.tuning_report()[0])
+            B.dancer(0, nmax, sb, coords, f=freqs, diskR=diskR, **kw)
+            new = [(k, v) for k, v in ctx.tuning_report()[0].items() if k not in before]
+            assert len(new) <= 1
+            return new[0] if new else None
+
+        ctx.set_option("autotune", 1)
+        short = key(5)
+        window = key(40)
+        assert short and window and " w" in window[0] and " w" not in short[0]
+        assert window[1][1:] == [0, 0]
+        assert key(60) is None  # the same window
+        other = key(40, diskR=0.1)
+        assert other and " w" in other[0] and other[1][1:] == [0, 0]
+        hist = key(12, returnsum=True, immediatesum=False)
+        assert hist and " w" not in hist[0]
+        with ctx.options(reduced=0):
+            assert key(40) is None  # the whole grid's entry of the short run
+
+    with ThreadPoolExecutor(max_workers=1) as ex:
+        ex.submit(run).result()
 
 
 def test_sweep_autotune_parseval_blocks():
