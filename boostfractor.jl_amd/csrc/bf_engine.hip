@@ -1695,6 +1695,16 @@ struct DancerPlan : DancerPlanBase {
                    : sizeof(cplx<S>) * (size_t)(band_hi - band_lo) * g.nx * 2 * R + ntab * (qtab ? K / 4 : K) * sizeof(cplx<C>);
             const size_t budget = (size_t)192 << 20;
             fb = (int)std::max<size_t>(1, budget / std::max<size_t>(touched, 1));
+            if (rd) {
+                // A window's batch is prepared on the whole grid: phase tables (and the reduced ones in full
+                // while they are formed) and the tilt/surface tables of every frequency, within 2 GB (1024^2,
+                // 20 tilted disks, a window of 41 rows: 32 frequencies, 192 MB of fields, would take 33 GB).
+                size_t nrough = 0;
+                for (int i = 0; i < R; i++)
+                    nrough += kind == BF_PROP_PROPAGATOR && (tx[i] != 0.0 || ty[i] != 0.0 || has_surf);
+                const size_t tables = sizeof(zd) * (ntab * (K + rsh.points()) + nrough * K);
+                fb = (int)std::max<size_t>(1, std::min<size_t>((size_t)fb, ((size_t)2 << 30) / tables));
+            }
         }
         fb = std::max(1, std::min(fb, std::min(nfreq, 64)));
         if (opt.freq_batch <= 0) {

@@ -83,6 +83,24 @@ def test_dancer_plans_batches_and_graphs(prec):
             plan.close()
 
 
+@pytest.mark.parametrize("tilted", [False, True])
+def test_dancer_batch_is_bounded_by_its_whole_grid_tables(tilted):
+    """a small window on a fine grid: the batch's phase and tilt tables are on the whole grid"""
+    n, R = 1024, 0.02
+    c = W.grid_coords(n)
+    sb = W.booster(c, ndisk=20, seed=15, flat=True)
+    nreg = len(sb.distance)
+    if tilted:
+        sb.relative_tilt_x = np.full(nreg, 1e-4)
+    f = np.linspace(19e9, 21e9, 64)
+    with B.context().options(reduced=1):
+        plan = B.DancerPlan(0, 9, sb, c, f, diskR=R)
+        fb = plan.freq_batch
+        plan.close()
+    tables = 16 * n * n * (20 + (nreg - 1 if tilted else 0))  # at least: 20 gaps of their own, tilts
+    assert 1 <= fb and fb * tables <= 2 << 30
+
+
 def test_history_amin_and_short_runs_keep_the_whole_grid():
     c = _grid(128, 128)
     sb = _booster(c, False, 14)
