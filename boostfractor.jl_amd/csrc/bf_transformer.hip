@@ -2994,24 +2994,24 @@ struct SeriesSlice {
 constexpr int SERIES_QMAX = 24;
 constexpr int SERIES_SLICE = 64;
 
-// weight table of the coefficient rows, wt[g][row0 + p] = exp(-1im*kz*c) * beta^p / p! * scale; zeros for
-// the groups [z0, z1)
+// weight table of the coefficient rows from r0 on, wt[g][row0 - r0 + p] = exp(-1im*kz*c) * beta^p / p! * scale;
+// zeros for the groups [z0, z1)
 __global__ void __launch_bounds__(256) k_series_coef(const SeriesKey* __restrict__ keys,
                                                      const double* __restrict__ gkx, const double* __restrict__ gky,
-                                                     int NG, int nrows, double scale, zd* __restrict__ wt, int z0,
-                                                     int z1) {
+                                                     int NG, int r0, int nrows, double scale,
+                                                     zd* __restrict__ wt, int z0, int z1) {
     const int g = blockIdx.x * blockDim.x + threadIdx.x;
     if (g >= NG) return;
     const SeriesKey k = keys[blockIdx.y];
+    zd* out = wt + (size_t)g * nrows + (k.row0 - r0);
     if (g >= z0 && g < z1) {
-        for (int p = 0; p < k.q; p++) wt[(size_t)g * nrows + k.row0 + p] = cmk<double>(0.0, 0.0);
+        for (int p = 0; p < k.q; p++) out[p] = cmk<double>(0.0, 0.0);
         return;
     }
     const zd kz = kz_of(k.k0sq, gkx[g], gky[g]);
     const zd e = kz_phase_of(kz, k.c);
     const zd beta = cmk<double>(kz.im * k.h, -kz.re * k.h);
     zd b = cmk<double>(e.re * scale, e.im * scale);
-    zd* out = wt + (size_t)g * nrows + k.row0;
     out[0] = b;
     for (int p = 1; p < k.q; p++) {
         b = cmul(b, beta);
@@ -3289,37 +3289,63 @@ struct Pack {
     T* at(size_t off) const { return reinterpret_cast<T*>(dev + off); }
 };
 
-// rows of the keys in order; returns their number
-static int number_rows(std::vector<SeriesKey>& keys) {
+// rows of the keys in order
+static void number_rows(std::vector<SeriesKey>& keys) {
     int nrows = 0;
     for (SeriesKey& k : keys) {
         k.row0 = nrows;
         nrows += k.q;
     }
-    return nrows;
+}
+
+// Weight tables hold as many rows at a time as TABLE_BYTES takes (at 1024^2, 131 000 groups, 244 of them; a
+// run's whole table fits up to 512^2 and some hundred gaps): the end of the part of the keys that starts at a,
+// and its rows.
+constexpr size_t TABLE_BYTES = (size_t)512 << 20;
+static size_t table_part(const std::vector<SeriesKey>& keys, size_t a, size_t NG, int& nrows) {
+    const int most = (int)std::min<size_t>((size_t)1 << 30, TABLE_BYTES / (sizeof(zd) * NG));
+    size_t b = a;
+    for (nrows = 0; b < keys.size() && (b == a || nrows + keys[b].q <= most); b++) nrows += keys[b].q;
+    return b;
+}
+// bytes of the largest part's table
+static size_t table_bytes(const std::vector<SeriesKey>& keys, size_t NG) {
+    size_t most = 0;
+    int nrows = 0;
+    for (size_t a = 0; NG > 0 && a < keys.size();) {
+        a = table_part(keys, a, NG, nrows);
+        most = std::max(most, (size_t)nrows);
+    }
+    return sizeof(zd) * NG * most;
 }
 
 // dst[row0 + p] = sum over the groups [g0, g1) of the keys' weights (k_series_coef) times H_g, the weights of
-// the groups [z0, z1) taken as zero (keys and dst on the device)
-static void table_product(bf_ctx* ctx, ModeCache& mc, int n, double scale, const SeriesKey* keys, size_t nkeys,
-                          zd* const* dst, int nrows, size_t g0, size_t g1, size_t z0, size_t z1) {
-    if (nkeys == 0 || g1 <= g0) return;
+// the groups [z0, z1) taken as zero (host: the keys, numbered; keys and dst on the device)
+static void table_product(bf_ctx* ctx, ModeCache& mc, int n, double scale, const std::vector<SeriesKey>& host,
+                          const SeriesKey* keys, zd* const* dst, size_t g0, size_t g1, size_t z0, size_t z1) {
+    if (host.empty() || g1 <= g0) return;
     hipStream_t s = ctx->stream;
     const size_t nn = (size_t)n * n, NG = g1 - g0;
-    DevBuf& dw = scratch_buf(ctx, SB_SW, sizeof(zd) * NG * (size_t)nrows);
-    {
-        TimedLaunch tl(ctx, "pseries", 0.0);
-        const int a = (int)(std::max(z0, g0) - g0), b = (int)(std::max(std::min(z1, g1), g0) - g0);
-        for (size_t k0 = 0; k0 < nkeys; k0 += 65535)
-            hipLaunchKernelGGL(k_series_coef,
-                               dim3((unsigned)((NG + 255) / 256), (unsigned)std::min<size_t>(65535, nkeys - k0)),
-                               dim3(256), 0, s, keys + k0, mc.gkx.as<double>() + g0, mc.gky.as<double>() + g0, (int)NG,
-                               nrows, scale, dw.as<zd>(), a, b);
-        BF_CHECK_LAUNCH();
+    zd* w = scratch_buf(ctx, SB_SW, table_bytes(host, NG)).as<zd>();
+    for (size_t a = 0, b = 0; a < host.size(); a = b) {
+        int nrows = 0;
+        b = table_part(host, a, NG, nrows);
+        const int r0 = host[a].row0;
+        {
+            TimedLaunch tl(ctx, "pseries", 0.0);
+            const int za = (int)(std::max(z0, g0) - g0), zb = (int)(std::max(std::min(z1, g1), g0) - g0);
+            for (size_t k0 = a; k0 < b; k0 += 65535)
+                hipLaunchKernelGGL(k_series_coef,
+                                   dim3((unsigned)((NG + 255) / 256), (unsigned)std::min<size_t>(65535, b - k0)),
+                                   dim3(256), 0, s, keys + k0, mc.gkx.as<double>() + g0, mc.gky.as<double>() + g0,
+                                   (int)NG, r0, nrows, scale, w, za, zb);
+            BF_CHECK_LAUNCH();
+        }
+        TimedLaunch tl(ctx, "pgemm", 8.0 * (double)parseval_cols(mc, nn) * (double)NG * (double)nrows);
+        launch_parseval_gemm<true>(ctx, parseval_wn(ctx, mc, nn, mc.gk2.size()), s, mc, nn, NG, nullptr, nullptr,
+                                   nullptr, nullptr, (size_t)nrows, scale, dst + r0, (nrows + PG_BM - 1) / PG_BM, w,
+                                   g0);
     }
-    TimedLaunch tl(ctx, "pgemm", 8.0 * (double)parseval_cols(mc, nn) * (double)NG * (double)nrows);
-    launch_parseval_gemm<true>(ctx, parseval_wn(ctx, mc, nn, mc.gk2.size()), s, mc, nn, NG, nullptr, nullptr, nullptr,
-                               nullptr, (size_t)nrows, scale, dst, (nrows + PG_BM - 1) / PG_BM, dw.as<zd>(), g0);
 }
 
 // ---------------------------------------------------------------------------
@@ -3576,7 +3602,7 @@ static void nodes_product(bf_ctx* ctx, ModeCache& mc, int n, double scale, std::
     }
     for (size_t i = 0; i < rows_a; i++) mat_a.push_back(mat + i * nn);
     for (size_t i = 0; i < rows_b; i++) mat_b.push_back(mat + (rows_a + i) * nn);
-    const int rows_near = number_rows(near);
+    number_rows(near);
     number_rows(na);
     number_rows(nb);
     Pack pk;
@@ -3584,13 +3610,14 @@ static void nodes_product(bf_ctx* ctx, ModeCache& mc, int n, double scale, std::
                  o_b = pk.add(nb), o_bd = pk.add(mat_b), o_t = pk.add(targets), o_s = pk.add(slices),
                  o_c = pk.add(coef);
     pk.upload(ctx, SB_NODES, st);
+    const size_t split = rows_b ? np.split : NG;
+    // one buffer for the three tables: one that grows would leave the smaller ones in the context's pool
+    scratch_buf(ctx, SB_SW, std::max({add ? table_bytes(near, np.d1 - np.d0) : 0, table_bytes(na, split),
+                                      table_bytes(nb, NG - split)}));
     if (add)
-        table_product(ctx, mc, n, scale, pk.at<SeriesKey>(o_near), near.size(), pk.at<zd*>(o_neard), rows_near, np.d0,
-                      np.d1, 0, 0);
-    table_product(ctx, mc, n, scale, pk.at<SeriesKey>(o_a), na.size(), pk.at<zd*>(o_ad), (int)rows_a, 0,
-                  rows_b ? np.split : NG, np.d0, np.d1);
-    table_product(ctx, mc, n, scale, pk.at<SeriesKey>(o_b), nb.size(), pk.at<zd*>(o_bd), (int)rows_b, np.split, NG,
-                  np.d0, np.d1);
+        table_product(ctx, mc, n, scale, near, pk.at<SeriesKey>(o_near), pk.at<zd*>(o_neard), np.d0, np.d1, 0, 0);
+    table_product(ctx, mc, n, scale, na, pk.at<SeriesKey>(o_a), pk.at<zd*>(o_ad), 0, split, np.d0, np.d1);
+    table_product(ctx, mc, n, scale, nb, pk.at<SeriesKey>(o_b), pk.at<zd*>(o_bd), split, NG, np.d0, np.d1);
     {
         TimedLaunch tl(ctx, "pseries", 4.0 * (double)nn * (double)targets.size() * q);
         for (size_t s0 = 0; s0 < slices.size(); s0 += 65535) {
@@ -3623,10 +3650,10 @@ static void series_form(bf_ctx* ctx, ModeCache& mc, int n, double scale, const s
         nodes_product(ctx, mc, n, scale, rest, rowdst, st);
         if (!rest.empty()) {
             Pack pk;
-            const int rows = number_rows(rest);
+            number_rows(rest);
             const size_t ok = pk.add(rest), od = pk.add(rowdst);
             pk.upload(ctx, SB_SKEY, st);
-            table_product(ctx, mc, n, scale, pk.at<SeriesKey>(ok), rest.size(), pk.at<zd*>(od), rows, 0, NG, 0, 0);
+            table_product(ctx, mc, n, scale, rest, pk.at<SeriesKey>(ok), pk.at<zd*>(od), 0, NG, 0, 0);
             if (!st) BF_HIP(hipStreamSynchronize(s));  // the host arrays go out of scope
         }
     }

@@ -6,6 +6,9 @@ k-bin groups, frequencies in any order and repeated, and gaps the
 interpolation has to leave alone: a lossy one and, with the propagator that
 keeps it, a permittivity with imaginary part +0.
 """
+import ctypes
+from concurrent.futures import ThreadPoolExecutor
+
 import numpy as np
 import pytest
 
@@ -46,3 +49,40 @@ def test_interpolated_products(engine_options, n, lo, hi, nf, kind):
             o = O.propagation_matrix(sb.distance[r], DISKR, sb.eps[r], 0.0, 0.0, np.zeros((n, n), dtype=complex),
                                      B.wavelength(freqs[q]), ocoords(coords), pat, kt, kind[1])
             assert rel(got[q][r], o) < 1e-10, (q, r)
+
+
+def test_weight_tables_are_bounded():
+    """a fine grid with many gaps: the interpolation's weight tables (131 000 groups x 40 gaps x 10 to 20
+    nodes, 0.8 GB in one) are formed in parts of 512 MB, and the parts add up"""
+    hip = ctypes.CDLL("libamdhip64.so")  # the runtime the library has loaded
+    coords = W.grid_coords(1024)
+    sb = W.booster(coords, ndisk=40, spacings=np.linspace(5e-3, 12e-3, 40), flat=True)
+    modes = _modes(coords, DISKR)
+    freqs = np.linspace(19.5e9, 20.5e9, 64)
+
+    def free_bytes():
+        f, t = ctypes.c_size_t(), ctypes.c_size_t()
+        assert hip.hipMemGetInfo(ctypes.byref(f), ctypes.byref(t)) == 0
+        return f.value
+
+    def run(nodes):
+        ctx = B.context()  # of a thread of its own
+        ctx.set_option("parseval_nodes", nodes)
+        before = free_bytes()
+        P = B.calc_propagation_matrices(sb, coords, modes, f=freqs, diskR=DISKR)
+        kept = before - free_bytes()
+        ctx.close()
+        return np.asarray([[P[q][r] for r in range(1, 81, 2)] for q in range(len(freqs))]), kept
+
+    def fresh(nodes):
+        with ThreadPoolExecutor(max_workers=1) as ex:
+            return ex.submit(run, nodes).result()
+
+    fresh(0)  # code objects and the runtime's own buffers
+    want, base = fresh(0)
+    got, kept = fresh(1)
+    assert np.any(got != want)  # (interpolated)
+    for q in range(len(freqs)):
+        for r in range(40):
+            assert rel(got[q][r], want[q][r]) < 1e-13, (q, r, rel(got[q][r], want[q][r]))
+    assert kept - base <= (512 << 20) + (128 << 20)
