@@ -157,6 +157,7 @@ int bf_ctx_create(int32_t device, bf_ctx** out) {
         BF_HIP(hipGetDeviceCount(&n));
         if (device < 0 || device >= n) throw bf::Error(BF_ERR_ARG, "device index out of range");
         BF_HIP(hipSetDevice(device));
+        c->pool->on_device(device);
         BF_HIP(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
         bf::noalloc_init(device);  // the allocation-free entry point's scratch address on this device
     });
@@ -237,6 +238,7 @@ static int64_t* option_slot(bf::EngineOptions& o, const char* name, int64_t& tmp
             return &tmp;
         }
     if (!strcmp(name, "batch_bytes")) return &o.batch_bytes;
+    if (!strcmp(name, "pool_mb")) return &o.pool_mb;
     return nullptr;
 }
 
@@ -246,9 +248,11 @@ int bf_ctx_set_option(bf_ctx* ctx, const char* name, int64_t value) {
     int* ip = nullptr;
     int64_t* slot = option_slot(ctx->opt, name, tmp, ip);
     BF_REQUIRE(ctx, slot != nullptr, BF_ERR_ARG, std::string("unknown option: ") + name);
-    BF_REQUIRE(ctx, value >= 0 && (!ip || value <= 1 << 30), BF_ERR_ARG, "option values must be >= 0");
+    const bool pool = slot == &ctx->opt.pool_mb;
+    BF_REQUIRE(ctx, value >= 0 && (!(ip || pool) || value <= 1 << 30), BF_ERR_ARG, "option values must be >= 0");
     if (ip) *ip = (int)value;
     else *slot = value;
+    if (pool) ctx->pool->limit((size_t)value << 20);
     return BF_OK;
 }
 

@@ -7,7 +7,6 @@
 #include <cstring>
 #include <map>
 #include <memory>
-#include <mutex>
 #include <stdexcept>
 #include <string>
 #include <utility>
@@ -15,15 +14,9 @@
 
 #include "../../include/boostfractor_hip.h"
 #include "bf_device.h"
+#include "bf_pool.h"
 
 namespace bf {
-
-// Internal failure carrying a C-ABI status code; converted to a return code at
-// the extern "C" boundary.
-struct Error : std::runtime_error {
-    int code;
-    Error(int c, const std::string& m) : std::runtime_error(m), code(c) {}
-};
 
 #define BF_HIP(call)                                                                                   \
     do {                                                                                               \
@@ -33,142 +26,6 @@ struct Error : std::runtime_error {
     } while (0)
 
 #define BF_CHECK_LAUNCH() BF_HIP(hipGetLastError())
-
-// Device memory given back by the buffers of one context, for its next ones.  A call
-// allocates a dozen buffers and frees them when it returns; hipMalloc and hipFree take
-// ~9 us each (milliseconds for hundreds of MB, and hipFree waits for the device).
-// Everything a context does is ordered on its one stream, so memory that work queued
-// earlier may still use can be handed out again at once.  The pool keeps at most
-// KEEP bytes (the last ones given back), frees them all when an allocation fails and
-// when the context is destroyed; blocks that come back later are freed directly.
-// A plan may be destroyed on another thread than its context's calls: the lock.
-class DevPool {
-  public:
-    static constexpr size_t KEEP = (size_t)2 << 30;
-    // block sizes: multiples of an eighth of the next lower power of two (at least 512 bytes)
-    static size_t round(size_t n) {
-        size_t g = 512;
-        while (g * 16 <= n) g *= 2;
-        return (n + g - 1) / g * g;
-    }
-    void* take(size_t block) {
-        std::lock_guard<std::mutex> lk(mu);
-        auto it = blocks.find(block);
-        if (it == blocks.end()) return nullptr;
-        void* p = it->second.first;
-        blocks.erase(it);
-        kept -= block;
-        return p;
-    }
-    void give(void* p, size_t block) {
-        std::vector<void*> out;
-        {
-            std::lock_guard<std::mutex> lk(mu);
-            if (closed || block > KEEP) {
-                out.push_back(p);
-            } else {
-                blocks.emplace(block, std::make_pair(p, ++turn));
-                kept += block;
-                while (kept > KEEP) {  // the block that lay unused longest goes
-                    auto old = std::min_element(blocks.begin(), blocks.end(), [](const auto& a, const auto& b) {
-                        return a.second.second < b.second.second;
-                    });
-                    out.push_back(old->second.first);
-                    kept -= old->first;
-                    blocks.erase(old);
-                }
-            }
-        }
-        for (void* q : out) (void)hipFree(q);
-    }
-    void trim(bool close = false) {
-        decltype(blocks) out;
-        {
-            std::lock_guard<std::mutex> lk(mu);
-            out.swap(blocks);
-            kept = 0;
-            closed = closed || close;
-        }
-        for (auto& b : out) (void)hipFree(b.second.first);
-    }
-    ~DevPool() { trim(true); }
-
-  private:
-    std::mutex mu;
-    std::multimap<size_t, std::pair<void*, uint64_t>> blocks;  // by size: address, turn it came back
-    size_t kept = 0;
-    uint64_t turn = 0;
-    bool closed = false;
-};
-// pool of the context whose call runs on this thread (null outside a call)
-const std::shared_ptr<DevPool>& call_pool();
-
-// Owning device allocation.
-struct DevBuf {
-    void* p = nullptr;
-    size_t bytes = 0;
-    DevBuf() = default;
-    explicit DevBuf(size_t n) { alloc(n); }
-    DevBuf(const DevBuf&) = delete;
-    DevBuf& operator=(const DevBuf&) = delete;
-    DevBuf(DevBuf&& o) noexcept : p(o.p), bytes(o.bytes), block(o.block), pool(std::move(o.pool)) {
-        o.p = nullptr;
-        o.bytes = 0;
-    }
-    DevBuf& operator=(DevBuf&& o) noexcept {
-        if (this != &o) {
-            release();
-            p = o.p;
-            bytes = o.bytes;
-            block = o.block;
-            pool = std::move(o.pool);
-            o.p = nullptr;
-            o.bytes = 0;
-        }
-        return *this;
-    }
-    ~DevBuf() { release(); }
-    void alloc(size_t n) {
-        release();
-        if (n == 0) return;
-        pool = call_pool();
-        block = pool ? DevPool::round(n) : n;
-        if (pool) p = pool->take(block);
-        if (!p) {
-            hipError_t e = hipMalloc(&p, block);
-            if (e == hipErrorOutOfMemory && pool) {  // what the pool keeps, and the rounding, may be what is missing
-                (void)hipGetLastError();
-                pool->trim();
-                block = n;
-                e = hipMalloc(&p, block);
-            }
-            if (e != hipSuccess) {
-                p = nullptr;
-                pool.reset();
-                throw Error(e == hipErrorOutOfMemory ? BF_ERR_NOMEM : BF_ERR_HIP,
-                            std::string("hipMalloc(") + std::to_string(n) + " bytes): " + hipGetErrorString(e));
-            }
-        }
-        bytes = n;
-    }
-    void release() {
-        if (p) {
-            if (pool)
-                pool->give(p, block);
-            else
-                (void)hipFree(p);
-        }
-        p = nullptr;
-        bytes = 0;
-        pool.reset();
-    }
-    template <typename U>
-    U* as() const { return static_cast<U*>(p); }
-
-  private:
-    size_t block = 0;  // bytes allocated
-    std::shared_ptr<DevPool> pool;
-};
 
 }  // namespace bf
 
@@ -214,6 +71,7 @@ struct EngineOptions {
     int pgemm_herm = 1;       // Parseval product over the upper triangles when the Grams are Hermitian
     int sinv_mfma = 1;        // inverse series on the matrix cores for 8 < n <= 32
     int autotune = 0;         // 1: time candidate launch shapes on first use of a shape key (kept per context)
+    int64_t pool_mb = (int64_t)(DevPool::KEEP >> 20);  // MiB of freed device memory kept for the next calls
     int64_t batch_bytes = 0;  // matrix budget of a sweep chunk (0: BF_DEFAULT_BATCH_BYTES)
 };
 // Options of the context whose call runs on this thread (defaults outside a call).

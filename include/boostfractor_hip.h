@@ -128,7 +128,11 @@ int bf_ctx_kernel_time(bf_ctx *ctx, const char *kernel, double *ms, int64_t *lau
  * "autotune" (below).  Shapes and budgets (0 = default): "col_tx", "rows"
  * (dancer launch shapes), "pg_wn" (2 or 4: Parseval product column blocks of
  * 128 or 256 matrix entries), "batch_bytes" (bytes of P and inv(P) per
- * chunk of a batched sweep; default 16 GiB).  Unknown names and negative
+ * chunk of a batched sweep; default 16 GiB).  "pool_mb": device memory that
+ * the context's calls and plans have freed is kept for the next ones, up to
+ * this many MiB (default 2048), until the context is destroyed or an
+ * allocation of any context on the device fails; 0 gives it all back at once
+ * and keeps none.  Unknown names and negative
  * values return BF_ERR_ARG.  No option changes a result beyond rounding. */
 int bf_ctx_set_option(bf_ctx *ctx, const char *name, int64_t value);
 int bf_ctx_get_option(bf_ctx *ctx, const char *name, int64_t *value);

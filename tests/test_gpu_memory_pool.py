@@ -97,3 +97,37 @@ def test_destroying_a_context_gives_its_memory_back():
     before, kept = used_by_a_context()
     assert free_bytes() >= before - (8 << 20)
     assert kept <= (2 << 30) + (64 << 20)
+
+
+def test_memory_given_back_on_request():
+    """option pool_mb: 0 frees what the context keeps and keeps nothing more; the results are the same"""
+    hip = ctypes.CDLL("libamdhip64.so")  # the runtime the library has loaded
+
+    def free_bytes():
+        f, t = ctypes.c_size_t(), ctypes.c_size_t()
+        assert hip.hipMemGetInfo(ctypes.byref(f), ctypes.byref(t)) == 0
+        return f.value
+
+    coords = W.grid_coords(256)
+    sb = W.booster(coords, ndisk=8, seed=93, flat=True)
+    ctx = B.Context()
+
+    def run():
+        plan = B.DancerPlan(0, 1, sb, coords, np.linspace(19e9, 21e9, 16), diskR=DISKR, ctx=ctx)
+        plan.run()
+        E = plan.fetch()[0]
+        plan.close()
+        return E
+
+    want = run()
+    ctx.set_option("pool_mb", 0)
+    empty = free_bytes()
+    assert np.array_equal(run(), want)
+    assert free_bytes() >= empty - (8 << 20)
+    ctx.set_option("pool_mb", 2048)
+    assert np.array_equal(run(), want)
+    kept = empty - free_bytes()
+    assert kept > 64 << 20  # 16 x 16 x 256^2 fields and their tables
+    ctx.set_option("pool_mb", 0)
+    assert free_bytes() >= empty - (8 << 20)
+    ctx.close()
