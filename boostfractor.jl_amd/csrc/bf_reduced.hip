@@ -72,12 +72,15 @@ __global__ void __launch_bounds__((RdCol<R>::NT)) __attribute__((amdgpu_waves_pe
     const uint32_t rowb = (uint32_t)Mx * SZ;
     const auto rf = buf_rsrc(a.F + d.off, (uint32_t)a.by * rowb);  // rows past the window read as zero
     const uint32_t o0 = ok && t < 16 ? (uint32_t)t * rowb + (uint32_t)x * SZ : BUF_OOB;
+    // byte offset of sample t + 16 m beyond o0, never past the field's end: what lies beyond the resource's
+    // length less this offset is out of range, and that difference is not to be negative
+    auto rows16 = [&](int m) { return (uint32_t)min(16 * m, a.by) * rowb; };
     const zd* tw = a.tw + (t < 16 ? t : 0);
     zd* s = sm + c;
     if (t < 16) {
         cplx<S> raw[H];
 #pragma unroll
-        for (int m = 0; m < H; m++) raw[m] = buf_load<S>(rf, o0, (uint32_t)(16 * m) * rowb);
+        for (int m = 0; m < H; m++) raw[m] = buf_load<S>(rf, o0, rows16(m));
         if (d.rtab >= 0 && ok) {  // uniform but for the last columns
             zd* q = a.sum + ((size_t)d.rtab * a.by + t) * Mx + x;
 #pragma unroll
@@ -140,7 +143,7 @@ __global__ void __launch_bounds__((RdCol<R>::NT)) __attribute__((amdgpu_waves_pe
         dft_out_half<R, true>(v);
 #pragma unroll
         for (int m = 0; m < H; m++)
-            buf_store<S>(rf, o0, ccast<S>(v[m]), (uint32_t)(16 * m) * rowb);
+            buf_store<S>(rf, o0, ccast<S>(v[m]), rows16(m));
     }
 }
 
