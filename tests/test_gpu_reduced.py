@@ -1,13 +1,14 @@
 """The bounce solvers on the aperture's window (circular convolutions of 16 R points per
 line) against the transforms of the whole grid: every radix, windows at the edge of a
 radix and of the grid, rectangular grids, tilts and surfaces, given emission and
-reflection, batches of frequencies, replayed graphs."""
+reflection, batches of frequencies, replayed graphs, k ranges without a mirror
+symmetry; and against the CPU oracle."""
 import numpy as np
 import pytest
 
 import BoostFractor as B
 from BoostFractor import workloads as W
-from helpers import DISKR, rel
+from helpers import DISKR, O, ocoords, osetup, rel
 
 pytestmark = pytest.mark.gpu
 # whole-grid and windowed transforms round differently by ~1e-15 per bounce; fields stored
@@ -63,6 +64,47 @@ def test_dancer_on_other_grids_and_windows(nx, ny, shift, prec):
         assert np.any(b != 0) and rel(a, b) < TOL[prec]
     a, b = _both(lambda: B.dancer(0, 8, sb, c, f=20e9, prop=B.propagatorNoTilts, diskR=DISKR, precision=prec))
     assert rel(a, b) < TOL[prec]
+
+
+def _shifted(c, kx, ky):
+    """k axes moved by fractions of a step: their phases are no longer even, the tables no quarters"""
+    k = lambda v, d: v + d * (v[1] - v[0])  # noqa: E731
+    return B.CoordinateSystem(c.X, c.Y, k(c.kX, kx), k(c.kY, ky))
+
+
+@pytest.mark.parametrize("nx,ny", [(128, 128), (101, 101), (128, 101)])
+@pytest.mark.parametrize("kx,ky", [(0.3, 0.0), (0.0, -0.4), (0.5, 0.2)])
+def test_k_ranges_without_mirror_symmetry(nx, ny, kx, ky):
+    c = _shifted(_grid(nx, ny), kx, ky)
+    sb = _booster(c, True, 16)
+    f = [19.9e9, 20.2e9]
+    a, b = _both(lambda: B.dancer(0, 9, sb, c, f=f, diskR=DISKR))
+    assert np.any(b != 0) and rel(a, b) < TOL["fp64"]
+    for q in range(len(f)):
+        assert rel(a[q], O.dancer(osetup(sb), ocoords(c), 0, 9, f[q], diskR=DISKR)) < 1e-10
+    sb.r[0] = 0.7 + 0.1j
+    for prec in ("fp64", "mixed"):
+        x, y = _both(lambda: B.cheerleader(0, 8, sb, c, f=f, diskR=DISKR, precision=prec, returnboth=True))
+        for u, v in zip(x, y):
+            assert np.any(v != 0) and rel(u, v) < TOL[prec]
+        if prec == "fp64":
+            for q in range(len(f)):
+                want = O.cheerleader(osetup(sb), ocoords(c), 0, 8, f[q], diskR=DISKR, returnboth=True)
+                assert all(rel(u[q], v) < 1e-10 for u, v in zip(x, want))
+
+
+@pytest.mark.parametrize("nx,ny,shift", [(128, 128, 0), (101, 130, 0), (256, 128, 30)])
+def test_window_matches_oracle(nx, ny, shift):
+    """symmetric k ranges (quarter tables), even and odd, a window off the centre: emission, reflection"""
+    c = _grid(nx, ny, shift)
+    sb = _booster(c, True, 17)
+    os_, oc = osetup(sb), ocoords(c)
+    refl = np.exp(-(c.X[None] ** 2 + c.Y[:, None] ** 2) / 0.1 ** 2) * np.exp(3j * c.X[None])
+    for kw in ({}, {"reflect": refl}):
+        got = B.dancer(0, 9, sb, c, f=20.1e9, diskR=DISKR, **kw)
+        assert rel(got, O.dancer(os_, oc, 0, 9, 20.1e9, diskR=DISKR, **kw)) < 1e-10
+        got = B.cheerleader(0, 8, sb, c, f=20.1e9, diskR=DISKR, **kw)
+        assert rel(got, O.cheerleader(os_, oc, 0, 8, 20.1e9, diskR=DISKR, **kw)) < 1e-10
 
 
 @pytest.mark.parametrize("prec", ["fp64", "mixed"])
