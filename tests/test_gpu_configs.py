@@ -27,11 +27,14 @@ def _beta2(E, coords):
     return W.beta2_dancer(E, coords, DISKR)
 
 
-def _plan(sb, coords, freqs, nmax, prec):
-    plan = B.DancerPlan(0, nmax, sb, coords, freqs, diskR=DISKR, precision=prec)
-    plan.run()
-    E, _ = plan.fetch()
-    plan.close()
+def _plan(sb, coords, freqs, nmax, prec, reduced=1):
+    """reduced=1, the default: bounces on the aperture's window, FP64 fields in both precisions; 0: on the
+    whole grid, fields stored in FP32 in mixed precision"""
+    with B.context().options(reduced=reduced):
+        plan = B.DancerPlan(0, nmax, sb, coords, freqs, diskR=DISKR, precision=prec)
+        plan.run()
+        E, _ = plan.fetch()
+        plan.close()
     return E
 
 
@@ -45,8 +48,9 @@ def test_config1_single_disk_in_full():
     want = O.dancer(osetup(sb), ocoords(coords), 0, 500, 20e9, O.PROP_PROPAGATOR, diskR=DISKR)
     assert rel(got, want) < TOL, rel(got, want)
     assert abs(_beta2(got, coords) / _beta2(want, coords) - 1) < TOL
-    plan = _plan(sb, coords, [20e9], 500, "fp64")
-    assert rel(plan[0], want) < TOL
+    for reduced in (0, 1):
+        plan = _plan(sb, coords, [20e9], 500, "fp64", reduced)
+        assert rel(plan[0], want) < TOL, reduced
 
 
 def test_config2_dancer_fp64_and_mixed_vs_oracle():
@@ -59,16 +63,17 @@ def test_config2_dancer_fp64_and_mixed_vs_oracle():
     freqs = np.linspace(19.5e9, 20.5e9, 50)
     nmax = 20
     print("config 2: dancer 256x256, 20 disks, 50 freqs, nmax=20 (fp64, mixed)", flush=True)
-    E64 = _plan(sb, coords, freqs, nmax, "fp64")
-    E32 = _plan(sb, coords, freqs, nmax, "mixed")
     os_, oc = osetup(sb), ocoords(coords)
     pick = [0, 37]
     want = pmap(lambda q: O.dancer(os_, oc, 0, nmax, freqs[q], O.PROP_PROPAGATOR, diskR=DISKR), pick)
-    for q, w in zip(pick, want):
-        assert rel(E64[q], w) < TOL, (q, rel(E64[q], w))
-        assert abs(_beta2(E32[q], coords) / _beta2(w, coords) - 1) < MIXED_TOL
-    err = np.abs(_beta2(E32, coords) / _beta2(E64, coords) - 1)
-    assert np.max(err) < MIXED_TOL, np.max(err)
+    for reduced in (0, 1):
+        E64 = _plan(sb, coords, freqs, nmax, "fp64", reduced)
+        E32 = _plan(sb, coords, freqs, nmax, "mixed", reduced)
+        for q, w in zip(pick, want):
+            assert rel(E64[q], w) < TOL, (reduced, q, rel(E64[q], w))
+            assert abs(_beta2(E32[q], coords) / _beta2(w, coords) - 1) < MIXED_TOL
+        err = np.abs(_beta2(E32, coords) / _beta2(E64, coords) - 1)
+        assert np.max(err) < MIXED_TOL, (reduced, np.max(err))
 
 
 def test_config2_full_size_mixed_vs_fp64():
@@ -80,10 +85,13 @@ def test_config2_full_size_mixed_vs_fp64():
     freqs = np.linspace(19.5e9, 20.5e9, 50)
     print("config 2: full size, 50 freqs, nmax=2000, mixed vs fp64", flush=True)
     b64 = _beta2(_plan(sb, coords, freqs, 2000, "fp64"), coords)
-    b32 = _beta2(_plan(sb, coords, freqs, 2000, "mixed"), coords)
-    err = np.abs(b32 / b64 - 1)
     assert np.all(np.isfinite(b64)) and np.min(b64) > 0
-    assert np.max(err) < MIXED_TOL, np.max(err)
+    for reduced in (0, 1):
+        b32 = _beta2(_plan(sb, coords, freqs, 2000, "mixed", reduced), coords)
+        err = np.abs(b32 / b64 - 1)
+        assert np.max(err) < MIXED_TOL, (reduced, np.max(err))
+    # the whole grid's FP64 passes
+    assert np.max(np.abs(_beta2(_plan(sb, coords, freqs, 2000, "fp64", 0), coords) / b64 - 1)) < TOL
 
 
 def _rough_512():
@@ -153,8 +161,8 @@ def test_config3_booster_chain_with_bessel_modes():
 
 
 def test_config4_dancer512_vs_oracle():
-    """configuration 4's booster at 512 x 512 (the three-pass register FFT and
-    the 512-point row pass) through the benchmark's plans over all 100
+    """configuration 4's booster at 512 x 512 (on the window, and on the whole grid with its
+    three-pass register FFT and 512-point row pass) through the benchmark's plans over all 100
     frequencies; the oracle checks frequencies 0 and 61 with nmax cut to 7
     (8 bounces, ~26 s of oracle per point): FP64 fields at 1e-10, mixed
     precision beta^2 at 1e-4"""
@@ -163,14 +171,15 @@ def test_config4_dancer512_vs_oracle():
     freqs = np.linspace(19.5e9, 20.5e9, 100)
     nmax = 7
     print("config 4: dancer 512x512, 20 disks, 100 freqs, nmax=7 (fp64, mixed)", flush=True)
-    E64 = _plan(sb, coords, freqs, nmax, "fp64")
-    E32 = _plan(sb, coords, freqs, nmax, "mixed")
     os_, oc = osetup(sb), ocoords(coords)
     pick = [0, 61]
     want = pmap(lambda q: O.dancer(os_, oc, 0, nmax, freqs[q], O.PROP_PROPAGATOR, diskR=DISKR), pick)
-    for q, w in zip(pick, want):
-        assert rel(E64[q], w) < TOL, (q, rel(E64[q], w))
-        assert abs(_beta2(E32[q], coords) / _beta2(w, coords) - 1) < MIXED_TOL
+    for reduced in (0, 1):
+        E64 = _plan(sb, coords, freqs, nmax, "fp64", reduced)
+        E32 = _plan(sb, coords, freqs, nmax, "mixed", reduced)
+        for q, w in zip(pick, want):
+            assert rel(E64[q], w) < TOL, (reduced, q, rel(E64[q], w))
+            assert abs(_beta2(E32[q], coords) / _beta2(w, coords) - 1) < MIXED_TOL
 
 
 def test_config4_full_nmax_mixed_vs_fp64():
@@ -181,9 +190,10 @@ def test_config4_full_nmax_mixed_vs_fp64():
     freqs = np.linspace(19.5e9, 20.5e9, 100)[[0, 33, 66, 99]]
     print("config 4: 512x512, 4 freqs, nmax=3000, mixed vs fp64", flush=True)
     b64 = _beta2(_plan(sb, coords, freqs, 3000, "fp64"), coords)
-    b32 = _beta2(_plan(sb, coords, freqs, 3000, "mixed"), coords)
-    err = np.abs(b32 / b64 - 1)
-    assert np.max(err) < MIXED_TOL, np.max(err)
+    for reduced in (0, 1):
+        b32 = _beta2(_plan(sb, coords, freqs, 3000, "mixed", reduced), coords)
+        err = np.abs(b32 / b64 - 1)
+        assert np.max(err) < MIXED_TOL, (reduced, np.max(err))
 
 
 # the sweep's geometries #395 (10 disks, 9 modes), #426 (45 disks, 15 modes), #132 (80 disks, 25 modes)

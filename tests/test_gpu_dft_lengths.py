@@ -57,15 +57,17 @@ def test_propagation_of_any_length(nx, ny, R):
 
 @pytest.mark.parametrize("n,prec", [(101, "fp64"), (101, "mixed"), (30, "fp64"), (52, "mixed"), (129, "fp64")])
 @pytest.mark.parametrize("rough", [False, True])
-def test_dancer_any_length_matches_direct_transforms(n, prec, rough):
+@pytest.mark.parametrize("reduced", [0, 1], ids=["grid", "window"])
+def test_dancer_any_length_matches_direct_transforms(n, prec, rough, reduced):
     """summed, history and amin runs against the direct transforms; skipping the
-    rows that the aperture zeroes changes no bit"""
+    rows that the aperture zeroes changes no bit (on the whole grid; the summed run's window, where the grid
+    has one, against the same direct transforms)"""
     coords = W.grid_coords(n)
     sb = W.rough_booster(coords, ndisk=2, seed=77) if rough else W.booster(coords, ndisk=3, seed=78)
     freqs = [19.8e9, 20.1e9, 20.3e9]
     out = {}
     for key, o in (("mm", {}), ("lds", {"fft_lds": 1}), ("rows", {"band": 0})):
-        with B.context().options(**o):
+        with B.context().options(reduced=reduced, **o):
             out[key] = [B.dancer(0, 12, sb, coords, f=freqs, diskR=DISKR, precision=prec),
                         B.dancer(0, 5, sb, coords, f=20e9, diskR=DISKR, precision=prec, returnsum=False,
                                  immediatesum=False),

@@ -17,6 +17,9 @@ from helpers import (DISKR, GOLDEN, O, deps_distance, ocoords, osetup, pmap, ref
 pytestmark = pytest.mark.gpu
 
 TOL = 1e-10
+# Summed bounces with amin = 0 run on the aperture's window from 8 bounces on (option reduced); the passes on
+# the whole grid serve history, amin, short runs and large apertures.  Tests of those passes run both ways.
+PATHS = pytest.mark.parametrize("reduced", [0, 1], ids=["grid", "window"])
 KINDS = [(B.propagator, O.PROP_PROPAGATOR), (B.propagatorNoTilts, O.PROP_NOTILTS),
          (B.propagator1D, O.PROP_1D), (B.propagatorMomentumSpace, O.PROP_MOMENTUM)]
 
@@ -72,8 +75,10 @@ def test_dancer_1d_golden():
     assert np.max(np.abs(np.array(got) / g - 1)) < TOL
 
 
-def test_dancer_3d_golden():
+@PATHS
+def test_dancer_3d_golden(engine_options, reduced):
     """test/runtests.jl:215 (3D dancer, nmax=200, Deps = 0:0.1:3pi), a spread of points."""
+    engine_options(reduced=reduced)
     coords = ref_coords()
     sb = ref_setup_eps9(coords)
     dx = ref_dx(coords)
@@ -85,8 +90,10 @@ def test_dancer_3d_golden():
         assert abs(b / g[i] - 1) < TOL, (i, b, g[i])
 
 
-def test_cheerleader_golden():
+@PATHS
+def test_cheerleader_golden(engine_options, reduced):
     """test/runtests.jl:211 (3D cheerleader, nmax=100), all 10 points."""
+    engine_options(reduced=reduced)
     coords = ref_coords()
     sb = ref_setup_default(coords)
     dx = ref_dx(coords)
@@ -99,9 +106,11 @@ def test_cheerleader_golden():
     assert np.max(np.abs(np.array(got) / g - 1)) < TOL
 
 
-def test_cheerleader_fine_golden():
+@PATHS
+def test_cheerleader_fine_golden(engine_options, reduced):
     """test/runtests.jl:212 (commented out; Deps = 0:0.1:3pi), a spread of points
     that are not on the :211 grid."""
+    engine_options(reduced=reduced)
     coords = ref_coords()
     sb = ref_setup_default(coords)
     dx = ref_dx(coords)
@@ -220,7 +229,8 @@ def test_cheerleader_amin_reflect():
 
 @pytest.mark.parametrize("prec", ["fp64", "mixed"])
 @pytest.mark.parametrize("N,ndisk,nmax", [(64, 3, 20), (128, 2, 9), (64, 1, 7), (64, 2, 0)])
-def test_cheerleader_wavefront_matches_sweep(prec, N, ndisk, nmax):
+@PATHS
+def test_cheerleader_wavefront_matches_sweep(prec, N, ndisk, nmax, reduced):
     """Steps of several iterations sharing launches (wavefront order) against the
     step-by-step sweep: the same kernels on the same fields in an order that
     keeps every dependency, so both outputs agree bit for bit (Nd = 4 and
@@ -228,7 +238,7 @@ def test_cheerleader_wavefront_matches_sweep(prec, N, ndisk, nmax):
     coords, sb = _small_booster(N=N, ndisk=ndisk, seed=1011 + N + ndisk)
     out = {}
     for wz in ("0", "1"):
-        with B.context().options(chwave=int(wz)):
+        with B.context().options(chwave=int(wz), reduced=reduced):
             out[wz] = B.cheerleader(0, nmax, sb, coords, f=[19.9e9, 20.05e9, 20.2e9], diskR=DISKR, precision=prec,
                                     returnboth=True)
     assert np.any(out["1"][1] != 0)
@@ -268,8 +278,11 @@ def test_cheerleader_emit_matches_oracle(prec, tol):
     assert rel(right, wr) < tol and rel(left, wl) < tol, (rel(right, wr), rel(left, wl))
 
 
-def test_dancer_mixed_precision_beta2():
-    """20-disk booster, 128^2, FP32 fields/FFT: beta^2 within 1e-4 of the FP64 engine."""
+@PATHS
+def test_dancer_mixed_precision_beta2(engine_options, reduced):
+    """20-disk booster, 128^2, fields stored in FP32 (on the whole grid; the window keeps FP64 ones): beta^2
+    within 1e-4 of the FP64 engine."""
+    engine_options(reduced=reduced)
     coords = W.grid_coords(128)
     sb = W.booster(coords, ndisk=20, seed=1000)
     freqs = np.linspace(19.5e9, 20.5e9, 6)
@@ -337,7 +350,8 @@ def test_dancer_row_band_is_exact(N, prec):
 @pytest.mark.parametrize("N,span,prec", [(128, 1.0, "fp64"), (128, 1.0, "mixed"), (128, 1.0, "fp32"),
                                          (128, 0.5, "fp64"), (128, 0.6, "mixed"), (256, 1.0, "mixed"),
                                          (256, 1.0, "fp64")])
-def test_dancer_pruned_transforms_match_unpruned(N, span, prec):
+@PATHS
+def test_dancer_pruned_transforms_match_unpruned(N, span, prec, reduced):
     """Band-pruned register transforms (butterflies of zero elements skipped,
     elements that are not stored not formed) against the unpruned ones: summed and
     history outputs, tilted and rough disks (tables applied in the row pass) and
@@ -349,7 +363,7 @@ def test_dancer_pruned_transforms_match_unpruned(N, span, prec):
     freqs = [19.8e9, 20.1e9]
     out = {}
     for prune in ("0", "1"):
-        with B.context().options(prune=int(prune)):
+        with B.context().options(prune=int(prune), reduced=reduced):
             e = B.dancer(0, 20, sb, coords, f=freqs, diskR=DISKR, precision=prec)
             h = B.dancer(0, 6, sb, coords, f=20e9, diskR=DISKR, precision=prec, returnsum=False, immediatesum=False)
             a = B.dancer(0.05, 40, sb, coords, f=20e9, diskR=DISKR, precision=prec)
@@ -366,15 +380,18 @@ def test_dancer_pruned_matches_oracle(N):
     against the oracle."""
     coords, sb = _small_booster(N=N, ndisk=2, seed=1004)
     freqs = [19.9e9, 20.2e9]
-    got = B.dancer(0, 15, sb, coords, f=freqs, diskR=DISKR)
     os_, oc = osetup(sb), ocoords(coords)
     want = pmap(lambda f: O.dancer(os_, oc, 0, 15, f, O.PROP_PROPAGATOR, diskR=DISKR), freqs)
-    for q in range(len(freqs)):
-        assert rel(got[q], want[q]) < TOL, (q, rel(got[q], want[q]))
+    for reduced in (0, 1):  # the pruned passes; the window, which has its own
+        with B.context().options(reduced=reduced):
+            got = B.dancer(0, 15, sb, coords, f=freqs, diskR=DISKR)
+        for q in range(len(freqs)):
+            assert rel(got[q], want[q]) < TOL, (reduced, q, rel(got[q], want[q]))
 
 
 @pytest.mark.parametrize("N,prec", [(64, "mixed"), (128, "mixed"), (128, "fp32"), (256, "mixed")])
-def test_dancer_quarter_tables_match_full(N, prec):
+@PATHS
+def test_dancer_quarter_tables_match_full(N, prec, reduced):
     """Complex64-field paths read quarter k-space tables ([N/2+1]^2 entries, a
     mirrored bin reads its mirror's phase, equal up to the rounding of the k
     range): against full tables within the storage rounding (1e-5 of the field
@@ -383,7 +400,7 @@ def test_dancer_quarter_tables_match_full(N, prec):
     freqs = [19.8e9, 20.1e9]
     out = {}
     for q in ("0", "1"):
-        with B.context().options(qtab=int(q)):
+        with B.context().options(qtab=int(q), reduced=reduced):
             out[q] = B.dancer(0, 20, sb, coords, f=freqs, diskR=DISKR, precision=prec)
     assert np.any(out["1"] != 0)
     tol = {"mixed": 1e-5, "fp32": 1e-4}[prec]
@@ -391,12 +408,14 @@ def test_dancer_quarter_tables_match_full(N, prec):
 
 
 @pytest.mark.parametrize("N,prec,amin", [(64, "fp64", 0.0), (128, "mixed", 0.0), (64, "mixed", 0.05)])
-def test_dancer_plan_graph_replays_match_eager(N, prec, amin):
+@PATHS
+def test_dancer_plan_graph_replays_match_eager(engine_options, N, prec, amin, reduced):
     """Plans replay each frequency batch's bounce loop from a HIP graph captured by
     the first run: three runs in a row, with eager work and synchronisations
     between them, each equal bit for bit to the plan launched bounce by bounce;
     5 frequencies in batches of 2 (three graphs, the last batch partial); the
     instrumented (timing) run takes the launch-by-launch path and agrees too."""
+    engine_options(reduced=reduced)
     coords, sb = _small_booster(N=N, ndisk=3, seed=1006)
     freqs = [19.7e9, 19.9e9, 20.0e9, 20.2e9, 20.4e9]
     with B.context().options(graph=0):
@@ -428,22 +447,27 @@ def test_cheerleader_band_matches_oracle():
     tilted and rough disks, both outputs, against the oracle."""
     coords, sb = _small_booster(N=128, ndisk=2, seed=1007)
     freqs = [19.9e9, 20.2e9]
-    left, right = B.cheerleader(0, 12, sb, coords, f=freqs, diskR=DISKR, returnboth=True)
+    out = {}
+    for reduced in (0, 1):  # the band's passes; the window, which has its own
+        with B.context().options(reduced=reduced):
+            out[reduced] = B.cheerleader(0, 12, sb, coords, f=freqs, diskR=DISKR, returnboth=True)
     os_, oc = osetup(sb), ocoords(coords)
     for q, f in enumerate(freqs):
         wl, wr = O.cheerleader(os_, oc, 0, 12, f, O.PROP_PROPAGATOR, diskR=DISKR, returnboth=True)
-        assert rel(right[q], wr) < TOL and rel(left[q], wl) < TOL, (q, rel(right[q], wr), rel(left[q], wl))
+        for reduced, (left, right) in out.items():
+            assert rel(right[q], wr) < TOL and rel(left[q], wl) < TOL, (reduced, q, rel(right[q], wr), rel(left[q], wl))
 
 
 @pytest.mark.parametrize("prec", ["fp64", "mixed"])
-def test_cheerleader_band_and_quarter_tables_match_full(prec):
+@PATHS
+def test_cheerleader_band_and_quarter_tables_match_full(prec, reduced):
     """Band-limited propagations (and, with complex64 fields, quarter phase
     tables) against every row and full tables: 1e-12 of the field maximum in
     FP64, 1e-5 with complex64 fields."""
     coords, sb = _small_booster(N=128, ndisk=3, seed=1008)
     out = {}
     for on in ("0", "1"):
-        with B.context().options(band=int(on), qtab=int(on)):
+        with B.context().options(band=int(on), qtab=int(on), reduced=reduced):
             out[on] = B.cheerleader(0, 20, sb, coords, f=[19.8e9, 20.1e9], diskR=DISKR, precision=prec)
     assert np.any(out["1"] != 0)
     tol = 1e-12 if prec == "fp64" else 1e-5
@@ -452,7 +476,8 @@ def test_cheerleader_band_and_quarter_tables_match_full(prec):
 
 @pytest.mark.parametrize("N", [64, 128])
 @pytest.mark.parametrize("prec", ["fp64", "mixed"])
-def test_cheerleader_fused_pair_rows_match_separate(prec, N):
+@PATHS
+def test_cheerleader_fused_pair_rows_match_separate(prec, N, reduced):
     """The pair steps' inverse row pass fused with the boundary update against the
     separate passes (tilted and rough disks, both outputs, amin criterion; with
     amin = 0 the fused pair steps keep the aperture band's rows only and store
@@ -461,7 +486,7 @@ def test_cheerleader_fused_pair_rows_match_separate(prec, N):
     coords, sb = _small_booster(N=N, ndisk=3, seed=1009)
     out = {}
     for fz, xf in (("0", "1"), ("1", "0"), ("1", "1")):
-        with B.context().options(chfuse=int(fz), chxf=int(xf)):
+        with B.context().options(chfuse=int(fz), chxf=int(xf), reduced=reduced):
             lr = B.cheerleader(0, 20, sb, coords, f=[19.8e9, 20.1e9], diskR=DISKR, precision=prec, returnboth=True)
             am = B.cheerleader(0.05, 40, sb, coords, f=20e9, diskR=DISKR, precision=prec)
         out[fz + xf] = (lr[0], lr[1], am)
