@@ -1317,10 +1317,21 @@ static bool k_mirrored(const double* k, int len) {
 // What a bounce solver on the window needs besides its fields: the window, the tables
 // of the reduced convolution and the whole-grid propagation of the sums.
 struct Reduced {
-    // Fewest bounces.  At 8 the window takes 1.85 against 2.99 ms (20 disks, 256^2, 8 frequencies), 0.44
-    // against 0.64 (10 disks, 101^2) and 5.6 against 8.6 (cheerleader, 256^2); a bounce costs 0.45 of the
-    // whole grid's, and the tables (two transforms of the grid each) are not spent on fewer.
+    // Fewest bounces.  At 8 the window takes 2.02 against 3.20 ms (dancer, 20 disks, 256^2, 8 frequencies) and
+    // 3.10 against 6.09 (cheerleader); a bounce costs 0.45 of the whole grid's, and the tables (two transforms
+    // of the grid each) are not spent on fewer.
     static constexpr int MIN_BOUNCES = 8;
+    // A dancer of few fields (directions x regions x frequencies) is bound by its launches on either path and
+    // needs more bounces to earn its tables back.  Window against whole grid at 8, 12 and 16 bounces, us a call:
+    // 6 fields of 128^2 332/296, 365/353, 396/431; 34 fields 341/323, 385/389, 422/465; 82 fields 378/379,
+    // 427/448, 461/533; 14 fields of 256^2 473/450, 519/539, 561/610; and of 34 fields of 101^2 317/299,
+    // 354/365, 386/429, 82 fields 372/382, 381/458, 424/560 (lengths that are no power of two cost the whole
+    // grid more).
+    static constexpr int MIN_BOUNCES_FEW = 11;
+    static bool few(const Grid& g, int64_t fields) {
+        const bool pow2 = !dft_length(g.nx) && !dft_length(g.ny);
+        return (double)fields * (double)g.K() < (pow2 ? 1.2e6 : 3.6e5);
+    }
     bf_ctx* ctx;
     const Grid* g;
     RdShape sh;
@@ -1351,7 +1362,7 @@ struct Reduced {
         return pow2 ? 4 * sh.points() <= 3 * g.K() : sh.points() <= g.K();
     }
     static bool usable(const Grid& g, int kind, double amin, int nmax, double diskR, RdShape& sh) {
-        return opts().reduced && use_reg_fft() && amin == 0.0 && nmax + 1 >= MIN_BOUNCES &&
+        return opts().reduced && use_reg_fft() && amin == 0.0 && nmax + 1 >= (opts().reduced == 2 ? 1 : MIN_BOUNCES) &&
                (kind == BF_PROP_PROPAGATOR || kind == BF_PROP_NOTILTS) && shape(g, diskR, sh);
     }
 
@@ -1548,10 +1559,17 @@ static bool quarter_tables_ok(const bf_coords* co, int kind) {
            (n & (n - 1)) == 0 && k_mirrored(co->kX, co->nx) && k_mirrored(co->kY, co->ny);
 }
 
-// Whether a dancer with FP64 arithmetic runs its bounces on the aperture's window (sh: its shape)
-static bool dancer_window(const Grid& g, int nreg, double amin, int nmax, int kind, double diskR,
-                          const DancerOptions& o, RdShape& sh) {
+// Whether a dancer with FP64 arithmetic could run its bounces on the aperture's window (sh: its shape)
+static bool dancer_has_window(const Grid& g, int nreg, double amin, int nmax, int kind, double diskR,
+                              const DancerOptions& o, RdShape& sh) {
     return o.window && (o.immediatesum || nmax == 0) && nreg > 2 && Reduced::usable(g, kind, amin, nmax, diskR, sh);
+}
+// and whether it does
+static bool dancer_window(const Grid& g, int nreg, double amin, int nmax, int nfr, int kind, double diskR,
+                          const DancerOptions& o, RdShape& sh) {
+    return dancer_has_window(g, nreg, amin, nmax, kind, diskR, o, sh) &&
+           (o.window == 2 || opts().reduced == 2 || nmax + 1 >= Reduced::MIN_BOUNCES_FEW ||
+            !Reduced::few(g, 2 * (int64_t)(nreg - 1) * nfr));
 }
 
 template <typename T>
@@ -1671,7 +1689,7 @@ struct DancerPlan : DancerPlanBase {
         nslices = opt.immediatesum ? 1 : nmax + 1;
         RdShape rsh;
         const bool rd =
-            std::is_same<T, double>::value && dancer_window(g, st->nreg, amin, nmax, kind, diskR, opt, rsh);
+            std::is_same<T, double>::value && dancer_window(g, st->nreg, amin, nmax, nfreq, kind, diskR, opt, rsh);
         const bool qtab = !rd && quarter_tables_ok<T>(co, kind);
         // Frequency batch: what one bounce of a batch touches (the band rows of every
         // field, plus one k-space table per distinct (eps, dz)) is kept near
@@ -2115,15 +2133,6 @@ struct DancerPlan : DancerPlanBase {
 static DancerPlanBase* make_dancer_plan_fixed(bf_ctx* ctx, const bf_setup* st, const bf_coords* co, double amin,
                                               int nmax, const double* fr, int nfr, int kind, double diskR,
                                               int precision, const DancerOptions& o) {
-    // On the window mixed precision keeps complex128 fields too: complex64 ones are 12% faster (the 20-disk
-    // booster, 256^2, 20 frequencies: 46.7 against 53.1 ms; 512^2, 4: 21.2 against 23.8) but round the
-    // emitted fields 0.7 to 1.35 times as far as the whole grid's mixed passes and their power up to twice.
-    if (precision == BF_PREC_MIXED) {
-        Grid g;
-        g.host(co);
-        RdShape sh;
-        if (dancer_window(g, st->nreg, amin, nmax, kind, diskR, o, sh)) precision = BF_PREC_FP64;
-    }
     if (precision == BF_PREC_MIXED) {
         auto* p = new DancerPlan<float>();
         try { p->init(ctx, st, co, amin, nmax, fr, nfr, kind, diskR, o); } catch (...) { delete p; throw; }
@@ -2169,7 +2178,7 @@ static void tune_dancer(bf_ctx* ctx, const bf_setup* st, const bf_coords* co, do
     base.graph = 0;
     base.returnsum = 1;
     base.immediatesum = 1;
-    base.window = window ? 1 : 0;  // (a summed run of a history plan stays on the whole grid)
+    base.window = window ? 2 : 0;  // whatever a shortened run's own path would be
     const int nm = std::min(nmax, TUNE_NMAX);
     // the heuristic batch, from a plan that picks it itself
     int fb0;
@@ -2235,12 +2244,18 @@ static void tune_dancer(bf_ctx* ctx, const bf_setup* st, const bf_coords* co, do
 DancerPlanBase* make_dancer_plan(bf_ctx* ctx, const bf_setup* st, const bf_coords* co, double amin, int nmax,
                                  const double* fr, int nfr, int kind, double diskR, int precision,
                                  const DancerOptions& o) {
+    Grid g;
+    g.host(co);
+    RdShape sh;
+    // Where there is a window mixed precision keeps complex128 fields too, on either path: on the window
+    // complex64 ones are 12% faster (the 20-disk booster, 256^2, 20 frequencies: 46.7 against 53.1 ms; 512^2, 4:
+    // 21.2 against 23.8) but round the emitted fields 0.7 to 1.35 times as far as the whole grid's mixed passes
+    // and their power up to twice.
+    if (precision == BF_PREC_MIXED && dancer_has_window(g, st->nreg, amin, nmax, kind, diskR, o, sh))
+        precision = BF_PREC_FP64;
     if (opts().autotune && o.freq_batch == 0 && o.col_tx == 0 && o.rows == 0 && nmax >= 1) {
-        Grid g;
-        g.host(co);
-        RdShape sh;
         const bool window =
-            precision != BF_PREC_FP32 && dancer_window(g, st->nreg, amin, nmax, kind, diskR, o, sh);
+            precision == BF_PREC_FP64 && dancer_window(g, st->nreg, amin, nmax, nfr, kind, diskR, o, sh);
         const std::string key = dancer_tune_key(co, st, precision, kind, amin, nfr, o, window, sh);
         if (!ctx->tuned.count(key))
             tune_dancer(ctx, st, co, amin, nmax, fr, nfr, kind, diskR, precision, o, window, key);

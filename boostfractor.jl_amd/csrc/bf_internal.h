@@ -51,7 +51,7 @@ struct EngineOptions {
     int prune = 1;            // band-pruned register transforms
     int qtab = 1;             // quarter k-space tables for complex64 fields
     int band = 1;             // skip the rows the aperture zeroes
-    int reduced = 1;          // bounce solvers on the aperture's window (amin 0, summed output)
+    int reduced = 1;          // bounce solvers on the aperture's window (amin 0, summed output; 2: however few bounces)
     int chfuse = 1;           // cheerleader: pair steps fused with their boundary update
     int chxf = 1;             // cheerleader: pair steps store the next masked row transform
     int chwave = 1;           // cheerleader: wavefront order when amin is 0
@@ -341,7 +341,7 @@ struct DancerOptions {
     int col_tx = 0, rows = 0;  // launch shapes (0: defaults)
     int band = 1;              // skip the rows the aperture zeroes (0: process every row)
     int graph = 0;             // replay each frequency batch's bounce loop from a captured HIP graph
-    int window = 1;            // bounces on the aperture's window where it serves (0: on the whole grid)
+    int window = 1;            // bounces on the aperture's window where it pays (0: never, 2: where there is one)
 };
 
 struct DancerPlanBase {

@@ -109,7 +109,8 @@ int bf_ctx_kernel_time(bf_ctx *ctx, const char *kernel, double *ms, int64_t *lau
  * register-resident ones), "prune" (band-pruned transforms), "qtab" (quarter
  * k-space tables for complex64 fields), "band" (skip the rows the aperture
  * zeroes), "reduced" (dancer and cheerleader with amin 0 and summed output:
- * bounces as circular convolutions on the aperture's window), "chfuse", "chxf", "chwave" (cheerleader pair fusion, stored row
+ * bounces as circular convolutions on the aperture's window, from 8 bounces
+ * on, dancers of few fields from 11; 2: however few), "chfuse", "chxf", "chwave" (cheerleader pair fusion, stored row
  * transforms, wavefront order), "graph" (dancer plans replay HIP graphs),
  * "parseval_groups", "disk_expansion", "parseval_series" (transformer work
  * reductions: k-bin groups, disks from the Gram matrix, air gaps by a series

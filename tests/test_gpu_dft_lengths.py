@@ -57,7 +57,7 @@ def test_propagation_of_any_length(nx, ny, R):
 
 @pytest.mark.parametrize("n,prec", [(101, "fp64"), (101, "mixed"), (30, "fp64"), (52, "mixed"), (129, "fp64")])
 @pytest.mark.parametrize("rough", [False, True])
-@pytest.mark.parametrize("reduced", [0, 1], ids=["grid", "window"])
+@pytest.mark.parametrize("reduced", [0, 2], ids=["grid", "window"])
 def test_dancer_any_length_matches_direct_transforms(n, prec, rough, reduced):
     """summed, history and amin runs against the direct transforms; skipping the
     rows that the aperture zeroes changes no bit (on the whole grid; the summed run's window, where the grid

@@ -17,9 +17,10 @@ from helpers import (DISKR, GOLDEN, O, deps_distance, ocoords, osetup, pmap, ref
 pytestmark = pytest.mark.gpu
 
 TOL = 1e-10
-# Summed bounces with amin = 0 run on the aperture's window from 8 bounces on (option reduced); the passes on
-# the whole grid serve history, amin, short runs and large apertures.  Tests of those passes run both ways.
-PATHS = pytest.mark.parametrize("reduced", [0, 1], ids=["grid", "window"])
+# Summed bounces with amin = 0 run on the aperture's window from 8 or 11 bounces on (option reduced; 2: always);
+# the passes on the whole grid serve history, amin, short runs and large apertures.  Tests of those passes run
+# both ways.
+PATHS = pytest.mark.parametrize("reduced", [0, 2], ids=["grid", "window"])
 KINDS = [(B.propagator, O.PROP_PROPAGATOR), (B.propagatorNoTilts, O.PROP_NOTILTS),
          (B.propagator1D, O.PROP_1D), (B.propagatorMomentumSpace, O.PROP_MOMENTUM)]
 
@@ -382,7 +383,7 @@ def test_dancer_pruned_matches_oracle(N):
     freqs = [19.9e9, 20.2e9]
     os_, oc = osetup(sb), ocoords(coords)
     want = pmap(lambda f: O.dancer(os_, oc, 0, 15, f, O.PROP_PROPAGATOR, diskR=DISKR), freqs)
-    for reduced in (0, 1):  # the pruned passes; the window, which has its own
+    for reduced in (0, 2):  # the pruned passes; the window, which has its own
         with B.context().options(reduced=reduced):
             got = B.dancer(0, 15, sb, coords, f=freqs, diskR=DISKR)
         for q in range(len(freqs)):
@@ -448,7 +449,7 @@ def test_cheerleader_band_matches_oracle():
     coords, sb = _small_booster(N=128, ndisk=2, seed=1007)
     freqs = [19.9e9, 20.2e9]
     out = {}
-    for reduced in (0, 1):  # the band's passes; the window, which has its own
+    for reduced in (0, 2):  # the band's passes; the window, which has its own
         with B.context().options(reduced=reduced):
             out[reduced] = B.cheerleader(0, 12, sb, coords, f=freqs, diskR=DISKR, returnboth=True)
     os_, oc = osetup(sb), ocoords(coords)

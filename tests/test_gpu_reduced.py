@@ -18,7 +18,7 @@ TOL = {"fp64": 1e-12, "mixed": 2e-6}
 
 def _both(fn):
     out = []
-    for on in (1, 0):
+    for on in (2, 0):  # 2: on the window however few the bounces
         with B.context().options(reduced=on):
             out.append(fn())
     return out
@@ -101,7 +101,8 @@ def test_window_matches_oracle(nx, ny, shift):
     os_, oc = osetup(sb), ocoords(c)
     refl = np.exp(-(c.X[None] ** 2 + c.Y[:, None] ** 2) / 0.1 ** 2) * np.exp(3j * c.X[None])
     for kw in ({}, {"reflect": refl}):
-        got = B.dancer(0, 9, sb, c, f=20.1e9, diskR=DISKR, **kw)
+        with B.context().options(reduced=2):
+            got = B.dancer(0, 9, sb, c, f=20.1e9, diskR=DISKR, **kw)
         assert rel(got, O.dancer(os_, oc, 0, 9, 20.1e9, diskR=DISKR, **kw)) < 1e-10
         got = B.cheerleader(0, 8, sb, c, f=20.1e9, diskR=DISKR, **kw)
         assert rel(got, O.cheerleader(os_, oc, 0, 8, 20.1e9, diskR=DISKR, **kw)) < 1e-10
@@ -112,7 +113,7 @@ def test_dancer_plans_batches_and_graphs(prec):
     c = _grid(128, 128)
     sb = _booster(c, True, 13)
     f = np.linspace(19.5e9, 20.5e9, 7)
-    want = B.dancer(0, 10, sb, c, f=f, diskR=DISKR, precision=prec)
+    want = B.dancer(0, 10, sb, c, f=f, diskR=DISKR, precision=prec)  # 11 bounces: on the window
     for graph in (0, 1):
         with B.context().options(graph=graph):
             plan = B.DancerPlan(0, 10, sb, c, f, diskR=DISKR, precision=prec, freq_batch=3)
@@ -143,15 +144,51 @@ def test_dancer_batch_is_bounded_by_its_whole_grid_tables(tilted):
     assert 1 <= fb and fb * tables <= 2 << 30
 
 
+def _by_rule(fn):
+    """the default's choice of the path, and the whole grid"""
+    out = []
+    for on in (1, 0):
+        with B.context().options(reduced=on):
+            out.append(fn())
+    return out
+
+
+@pytest.mark.parametrize("n,ndisk,nfreq,window_from", [(128, 1, 1, 11), (101, 3, 1, 11), (256, 2, 1, 11),
+                                                       (128, 9, 2, 8), (101, 9, 1, 8), (256, 9, 1, 8)])
+@pytest.mark.parametrize("prec", ["fp64", "mixed"])
+def test_few_fields_take_the_window_later(n, ndisk, nfreq, window_from, prec):
+    """8 to 10 bounces of few fields are faster on the whole grid; with the same FP64 fields"""
+    c = W.grid_coords(n)
+    sb = W.booster(c, ndisk=ndisk, seed=18)
+    f = np.linspace(19.9e9, 20.1e9, nfreq)
+    for nmax in (6, 7, 9, 10, 14):
+        with B.context().options(reduced=0):
+            grid = B.dancer(0, nmax, sb, c, f=f, diskR=DISKR, precision="mixed" if nmax == 6 else "fp64")
+        got = B.dancer(0, nmax, sb, c, f=f, diskR=DISKR, precision="mixed" if nmax == 6 else prec)
+        assert rel(got, grid) < TOL["fp64"]
+        assert np.array_equal(got, grid) == (nmax + 1 < window_from)
+
+
+def test_short_runs_on_the_window():
+    """option reduced=2: one, two and four bounces"""
+    c = _grid(128, 101)
+    sb = _booster(c, True, 19)
+    for nmax in (0, 1, 3):
+        for fn in (lambda: B.dancer(0, nmax, sb, c, f=[19.9e9, 20.1e9], diskR=DISKR),
+                   lambda: B.cheerleader(0, nmax, sb, c, f=[19.9e9, 20.1e9], diskR=DISKR)):
+            a, b = _both(fn)
+            assert np.any(b != 0) and rel(a, b) < TOL["fp64"]
+
+
 def test_history_amin_and_short_runs_keep_the_whole_grid():
     c = _grid(128, 128)
     sb = _booster(c, False, 14)
     for kw in ({"returnsum": False, "immediatesum": False}, {"returnsum": True, "immediatesum": False}):
-        a, b = _both(lambda: B.dancer(0, 9, sb, c, f=20e9, diskR=DISKR, **kw))
+        a, b = _by_rule(lambda: B.dancer(0, 9, sb, c, f=20e9, diskR=DISKR, **kw))
         assert np.array_equal(a, b)
-    a, b = _both(lambda: B.dancer(0.05, 30, sb, c, f=20e9, diskR=DISKR))
+    a, b = _by_rule(lambda: B.dancer(0.05, 30, sb, c, f=20e9, diskR=DISKR))
     assert np.array_equal(a, b)
-    a, b = _both(lambda: B.dancer(0, 3, sb, c, f=20e9, diskR=DISKR))
+    a, b = _by_rule(lambda: B.dancer(0, 3, sb, c, f=20e9, diskR=DISKR))
     assert np.array_equal(a, b)
 
 
@@ -177,7 +214,7 @@ def test_cheerleader_on_the_window(nx, ny, shift, prec, ndisk):
 def test_cheerleader_amin_and_short_runs_keep_the_whole_grid():
     c = _grid(128, 128)
     sb = _booster(c, False, 22)
-    a, b = _both(lambda: B.cheerleader(0.05, 30, sb, c, f=20e9, diskR=DISKR))
+    a, b = _by_rule(lambda: B.cheerleader(0.05, 30, sb, c, f=20e9, diskR=DISKR))
     assert np.array_equal(a, b)
-    a, b = _both(lambda: B.cheerleader(0, 2, sb, c, f=20e9, diskR=DISKR))
+    a, b = _by_rule(lambda: B.cheerleader(0, 2, sb, c, f=20e9, diskR=DISKR))
     assert np.array_equal(a, b)
