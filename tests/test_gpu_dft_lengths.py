@@ -98,6 +98,19 @@ def test_cheerleader_any_length_matches_direct_transforms(n, prec, opt):
         assert np.any(w != 0) and rel(g, w) < tol
 
 
+@pytest.mark.parametrize("n,direct", [(7, True), (24, True), (31, True), (33, False)])
+def test_short_lines_with_the_amin_criterion(n, direct):
+    """one region at a time on lines below 32 points: the direct sums in LDS, bit for bit"""
+    coords = W.grid_coords(n)
+    sb = W.rough_booster(coords, ndisk=2, seed=81)
+    out = []
+    for lds in (0, 1):
+        with B.context().options(fft_lds=lds):
+            out.append(B.cheerleader(1e-6, 12, sb, coords, f=[19.8e9, 20.1e9], diskR=0.3))
+    assert np.any(out[1] != 0) and rel(out[0], out[1]) < 1e-12
+    assert np.array_equal(out[0], out[1]) == direct
+
+
 def test_empty_aperture_gives_a_zero_field():
     c = _coords(30, 21)
     c.X[:] += 0.5 / 30  # no sample at the centre
