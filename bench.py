@@ -12,8 +12,8 @@ whole sweep once; `value` is the whole sweep's points over the timed time.
 The sweep has no reduced-precision path (its products run on FP64 MFMA), so
 `mixed_over_fp64` is 1.0.  The dancer workloads (`--workload dancer`,
 `dancer512`) time the mixed path against FP64 and report the ratio and the
-beta^2 error of every point (bounces on the aperture's window keep complex128
-fields in both).
+beta^2 error of every point (on these sizes both keep complex128 fields on the
+aperture's window).
 
 Kernel timing: the timed steps run without instrumentation; one more step
 then records HIP events on the engine's stream around every launch of the

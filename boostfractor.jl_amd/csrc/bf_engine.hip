@@ -1695,7 +1695,10 @@ struct DancerPlan : DancerPlanBase {
         // field, plus one k-space table per distinct (eps, dz)) is kept near
         // 192 MB, the size of the Infinity Cache; the frequencies are then spread
         // evenly over the batches.  Measured on the 20-disk booster at 256^2:
-        // 5 frequencies (complex64 fields) and 4 (complex128) are the fastest.
+        // 5 frequencies (complex64 fields) and 4 (complex128) are the fastest.  On the
+        // window the rule gives 10 at 256^2 (40 frequencies x 201 bounces 104.3 ms; 5: 114.1,
+        // 14: 105.4, 20: 123.0), 2 at 512^2 (16 x 101: 90.0; 3: 88.6, 4: 93.2), 30 of 60 at
+        // 128^2 (41.1; 20: 43.4, 60: 43.3) and all 60 at 101^2 (25.6; 30: 27.7).
         const size_t per = sizeof(cplx<S>) * K * 2 * R;
         if (opt.freq_batch > 0) {
             fb = opt.freq_batch;

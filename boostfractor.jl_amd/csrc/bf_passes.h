@@ -28,7 +28,7 @@ template <> struct Compute<f32pure> { using type = float; };
 
 // The matrix-core line transforms of a pass (bf_dftmm.h)
 struct DftArgs {
-    const double2* tab = nullptr;  // (cos, sin)(2 pi a b / n), [dft_ld(n)][dft_ld(n)]
+    const double2* tab = nullptr;  // (cos, sin)(2 pi a b / n), [dft_tab_rows(n)][dft_ld(n)]
     int lo = 0;                    // smallest folded index inside the aperture along the line
     int smax = 1;                  // waves that may share an output tile (set by the launcher)
 };

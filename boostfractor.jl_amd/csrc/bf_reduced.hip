@@ -56,10 +56,11 @@ __device__ __forceinline__ void rd_store(cplx<double>* f, int k1, const zd (&v)[
 
 // Column pass: transform along y, times the table, and back, window rows in and out.
 // Threads (t, column) for the samples, (k1, column) for the wavenumbers; neighbouring
-// lanes are neighbouring columns, in HBM and in LDS.  VALU-bound in FP64 arithmetic:
-// 630 instructions per lane at R = 10 for 16 (10) lanes a line.  With the row pass, 20 disks
-// on 256^2 (20 frequencies x 201 bounces) take 53 ms against 82 on the whole grid, 512^2 (4 x
-// 101) 24 against 52; 3 disks on 101^2 (16 x 201) 3.7 against 9.2.
+// lanes are neighbouring columns, in HBM and in LDS.  Bound by the traffic behind L2: 10 frequencies
+// of 20 disks on 256^2 (R = 10) move 464 MB, 323 of them the fields, in 74 us, 6.3 TB/s, with FP64
+// issue at 0.41 and LDS at 0.25 of the time (the row pass: 322 MB in 54 us, FP64 issue 0.36).  Both
+// passes, 20 disks on 256^2 (20 frequencies x 201 bounces), take 53 ms against 82 on the whole grid,
+// 512^2 (4 x 101) 24 against 52; 3 disks on 101^2 (16 x 201) 3.7 against 9.2.
 template <typename S, int R>
 __global__ void __launch_bounds__((RdCol<R>::NT)) __attribute__((amdgpu_waves_per_eu(RdCol<R>::WPE))) k_rd_cols(RdColArgs<S> a) {
     constexpr int C = RdCol<R>::C, H = rd_half(R);

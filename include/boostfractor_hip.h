@@ -50,7 +50,9 @@ extern "C" {
 /* arithmetic of the hot path */
 #define BF_PREC_FP64 0  /* everything in FP64 */
 #define BF_PREC_MIXED 1 /* fields stored in FP32 in HBM, in-register FFT/phase/update arithmetic in FP64,
-                           FP64 outputs and transfer-matrix chains */
+                           FP64 outputs and transfer-matrix chains; FP64 fields in dancers of at least 8
+                           bounces with amin 0 and summed output whose aperture has a window (see option
+                           "reduced" below) */
 #define BF_PREC_FP32 2  /* FP32 storage and FP32 arithmetic (accuracy study; not the mixed path) */
 
 #define BF_MAX_GRID 1024
