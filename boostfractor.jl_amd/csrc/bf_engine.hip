@@ -1624,6 +1624,7 @@ struct DancerPlan : DancerPlanBase {
         BF_HIP(hipEventSynchronize(ev[((size_t)(nb_bounces - 1) * 2 + 0) * 2 + 1]));
         for (int n = 0; n < nb_bounces; n++)
             for (int k = 0; k < 2; k++) {
+                if (red && k == 0 && n == nb_bounces - 1) continue;  // the last bounce has no boundaries there
                 float m = 0.f;
                 BF_HIP(hipEventElapsedTime(&m, ev[((size_t)n * 2 + k) * 2], ev[((size_t)n * 2 + k) * 2 + 1]));
                 ms[k] += m;

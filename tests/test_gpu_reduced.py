@@ -126,6 +126,20 @@ def test_dancer_plans_batches_and_graphs(prec):
             plan.close()
 
 
+def test_plan_timing_counts_the_launches():
+    c = _grid(128, 128)
+    sb = _booster(c, False, 20)
+    for reduced, rows in ((0, 12), (1, 11)):  # the window's last bounce ends with the sum of the exit fields
+        with B.context().options(reduced=reduced):
+            plan = B.DancerPlan(0, 11, sb, c, np.linspace(19.8e9, 20.2e9, 6), diskR=DISKR, freq_batch=3)
+            plan.timing(True)
+            plan.run()
+            kt = plan.kernel_times()
+            plan.close()
+        assert kt["col_pass"][1] == 2 * 12 and kt["row_pass"][1] == 2 * rows
+        assert kt["col_pass"][0] > 0 and kt["row_pass"][0] > 0
+
+
 @pytest.mark.parametrize("tilted", [False, True])
 def test_dancer_batch_is_bounded_by_its_whole_grid_tables(tilted):
     """a small window on a fine grid: the batch's phase and tilt tables are on the whole grid"""
